@@ -931,7 +931,8 @@ static void launch_residual64(const Mat& M, const TV* vals, const double* b, con
                               CgState* st, hipStream_t s) {
   const int grid = row_grid(M.a, M.a.fmt != MIFE_FMT_CSR ? 64 : M.L);
   const int tk = prof::begin(s);
-  MIFE_DISPATCH_FMT(M.a, M.L, (residual64_kernel<FMT_, L_, TV><<<grid, 256, 0, s>>>(M.a, vals, b, x, r, st)));
+  MIFE_DISPATCH_FMT(M.a, M.L, (residual64_kernel<FMT_, L_, TV><<<grid, 256, 0, s>>>(read_once(M.a), vals, b, x, r,
+                                                                                        st)));
   prof::end(tk, s, prof::kResidual64);
   fin_residual_kernel<<<1, kFinThreads, 0, s>>>(st, grid);
 }

@@ -9,8 +9,11 @@
 //    so every value/column load of the wavefront is one coalesced 256-byte
 //    access and no row pointer is read per row.  Column indices are in the
 //    permuted (slice) numbering, so the CG vectors live in that numbering too.
-// Values and columns are read once per product and streamed past the caches
-// with non-temporal loads; the gathered vector stays cache-resident.
+// Values and columns are read once per product.  A Krylov solve reads them again
+// in every iteration, so as much of them as the memory-side Infinity Cache
+// (256 MB) holds is read with plain loads and served from there, and the rest is
+// streamed past it with non-temporal loads (keep_sixteenths below); the gathered
+// vector stays in L2.
 #pragma once
 #include "mife_common.hpp"
 #include <algorithm>
@@ -49,7 +52,23 @@ struct MatArgs {
   const int32_t* order;  // SELL schedule (8 ranges of `span` slices, -1 padded) or null
   int span;
   int split;  // scheduled SELL: wavefronts per slice (1, 2 or 4)
+  int keep64, keep32;  // SELL: sixteenths of the slices read with plain loads (FP64, FP32 values)
 };
+
+// Sixteenths of a matrix of `bytes` (values and columns) that repeated products
+// read with plain loads, which the Infinity Cache keeps between products; the
+// other slices' non-temporal loads pass it by.  A matrix within kCacheBytes is
+// kept whole.  Measured: FP64 CG on a 96x32x32 elasticity system (200 MB of node
+// blocks) 73.4 ms all non-temporal, 62.3 ms kept whole; GMRES on a 12^3 Q2/Q1
+// Newton matrix (89 MB) 59.8 -> 53.9 ms, MINRES on its FP32 values 45.8 -> 39.0 ms;
+// a 326 MB FP32 matrix (48^3 triquadratic diffusion, whole pass) 41.3 ms all
+// non-temporal, 44.9 ms all plain (it evicts itself), 37.4 ms with 10 sixteenths
+// kept.  Kept bytes of 180 to 220 MB measured within 0.2% of each other there, 140
+// and 240 MB 1% slower.
+constexpr double kCacheBytes = 2.1e8;
+inline int keep_sixteenths(double bytes) {
+  return bytes <= kCacheBytes ? 16 : (int)(16.0 * kCacheBytes / bytes);
+}
 
 // Shape of a SELL3 descriptor: three rows per node row, ceil(node rows / 64)
 // slices, 16-bit node columns.
@@ -66,14 +85,37 @@ inline MatArgs mat_args(const mife_matrix* A) {
   const bool sell = A->format == MIFE_FMT_SELL || sell3;
   const bool c16 = sell && A->col_base != nullptr;
   const bool sched = sell && A->slice_order != nullptr && A->order_span > 0;
+  // column bytes per stored value (SELL3: one 16-bit column per nine values)
+  const double cb = sell3 ? 2.0 / 9.0 : (c16 ? 2.0 : 4.0);
   return MatArgs{A->n, sell3 ? kFmtSell3 : (c16 ? kFmtSell16 : A->format), A->ptr, A->col, A->n_slices,
                  c16 ? A->col_base : nullptr, sched ? A->slice_order : nullptr, sched ? A->order_span : 0,
-                 sched ? sell_split(A->n_slices) : 1};
+                 sched ? sell_split(A->n_slices) : 1, keep_sixteenths((8.0 + cb) * (double)A->nnz),
+                 keep_sixteenths((4.0 + cb) * (double)A->nnz)};
+}
+
+// A matrix that is read once (a residual between other products): nothing kept.
+inline MatArgs read_once(MatArgs A) {
+  A.keep64 = A.keep32 = 0;
+  return A;
 }
 
 template <typename T>
 __device__ __forceinline__ T stream_load(const T* p) {
   return __builtin_nontemporal_load(p);
+}
+
+// Matrix loads: NT streams past the Infinity Cache.
+template <bool NT, typename T>
+__device__ __forceinline__ T mat_load(const T* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+
+// Whether slot (or slice) k is one of the kept slices: every XCD's range and every
+// stretch of time then mixes kept and streamed slices.
+template <typename TV>
+__device__ __forceinline__ bool slice_kept(const MatArgs& A, int k) {
+  return (k & 15) < (sizeof(TV) == 8 ? A.keep64 : A.keep32);
 }
 
 template <typename T, int L>
@@ -113,7 +155,7 @@ __device__ __forceinline__ T row_partial(const int32_t* __restrict__ rp, const i
 
 // SELL-64 row sum of slice `s`, lane `lane` (one row per lane, complete sum),
 // eight entries in flight per lane.
-template <typename T, typename TV = T>
+template <typename T, typename TV = T, bool NT = true>
 __device__ __forceinline__ T sell_row(const int32_t* __restrict__ sp, const int32_t* __restrict__ col,
                                       const TV* __restrict__ vals, const T* __restrict__ x, int s, int lane) {
   const int base = sp[s];
@@ -126,9 +168,9 @@ __device__ __forceinline__ T sell_row(const int32_t* __restrict__ sp, const int3
     int ci[8];
     TV vi[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) ci[u] = stream_load(c + u * kSlice);
+    for (int u = 0; u < 8; ++u) ci[u] = mat_load<NT>(c + u * kSlice);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) vi[u] = stream_load(v + u * kSlice);
+    for (int u = 0; u < 8; ++u) vi[u] = mat_load<NT>(v + u * kSlice);
     a0 += vi[0] * x[ci[0]];
     a1 += vi[1] * x[ci[1]];
     a2 += vi[2] * x[ci[2]];
@@ -141,7 +183,7 @@ __device__ __forceinline__ T sell_row(const int32_t* __restrict__ sp, const int3
     v += 8 * kSlice;
   }
   for (; j < len; ++j) {
-    a0 += (T)stream_load(v) * x[stream_load(c)];
+    a0 += (T)mat_load<NT>(v) * x[mat_load<NT>(c)];
     c += kSlice;
     v += kSlice;
   }
@@ -150,7 +192,7 @@ __device__ __forceinline__ T sell_row(const int32_t* __restrict__ sp, const int3
 
 // As sell_row with 16-bit columns relative to the slice's base column; eight
 // entries in flight per lane (the 2-byte columns leave registers for it).
-template <typename T, typename TV = T>
+template <typename T, typename TV = T, bool NT = true>
 __device__ __forceinline__ T sell16_row(const int32_t* __restrict__ sp, const uint16_t* __restrict__ col,
                                         const int32_t* __restrict__ cbase, const TV* __restrict__ vals,
                                         const T* __restrict__ x, int s, int lane) {
@@ -165,9 +207,9 @@ __device__ __forceinline__ T sell16_row(const int32_t* __restrict__ sp, const ui
     int ci[8];
     TV vi[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) ci[u] = stream_load(c + u * kSlice);
+    for (int u = 0; u < 8; ++u) ci[u] = mat_load<NT>(c + u * kSlice);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) vi[u] = stream_load(v + u * kSlice);
+    for (int u = 0; u < 8; ++u) vi[u] = mat_load<NT>(v + u * kSlice);
     a0 += vi[0] * xs[ci[0]];
     a1 += vi[1] * xs[ci[1]];
     a2 += vi[2] * xs[ci[2]];
@@ -180,7 +222,7 @@ __device__ __forceinline__ T sell16_row(const int32_t* __restrict__ sp, const ui
     v += 8 * kSlice;
   }
   for (; j < len; ++j) {
-    a0 += (T)stream_load(v) * xs[(int)stream_load(c)];
+    a0 += (T)mat_load<NT>(v) * xs[(int)mat_load<NT>(c)];
     c += kSlice;
     v += kSlice;
   }
@@ -191,7 +233,7 @@ __device__ __forceinline__ T sell16_row(const int32_t* __restrict__ sp, const ui
 // entries start at `base`, `len` per row, base column cb (16-bit columns): the
 // wavefront takes chunks h, h + W, h + 2W, ... of eight entries; with W = 1 the
 // order of the additions is that of sell_row / sell16_row.
-template <typename T, bool C16, typename TV = T>
+template <typename T, bool C16, typename TV, bool NT>
 __device__ __forceinline__ T sell_row_part(const MatArgs& A, const TV* __restrict__ vals, const T* __restrict__ x,
                                            int base, int len, int cb, int lane, int h, int W) {
   constexpr int D = 8;
@@ -200,8 +242,8 @@ __device__ __forceinline__ T sell_row_part(const MatArgs& A, const TV* __restric
   const int32_t* c32 = A.col + base + lane;
   const TV* v = vals + base + lane;
   auto col = [&](int j) -> int {
-    if constexpr (C16) return (int)stream_load(c16 + j * kSlice);
-    else return stream_load(c32 + j * kSlice);
+    if constexpr (C16) return (int)mat_load<NT>(c16 + j * kSlice);
+    else return mat_load<NT>(c32 + j * kSlice);
   };
   T a0 = 0, a1 = 0, a2 = 0, a3 = 0;
   int j = h * D;
@@ -211,7 +253,7 @@ __device__ __forceinline__ T sell_row_part(const MatArgs& A, const TV* __restric
 #pragma unroll
     for (int u = 0; u < D; ++u) ci[u] = col(j + u);
 #pragma unroll
-    for (int u = 0; u < D; ++u) vi[u] = stream_load(v + (j + u) * kSlice);
+    for (int u = 0; u < D; ++u) vi[u] = mat_load<NT>(v + (j + u) * kSlice);
     a0 += vi[0] * xs[ci[0]];
     a1 += vi[1] * xs[ci[1]];
     a2 += vi[2] * xs[ci[2]];
@@ -221,7 +263,7 @@ __device__ __forceinline__ T sell_row_part(const MatArgs& A, const TV* __restric
     a2 += vi[6] * xs[ci[6]];
     a3 += vi[7] * xs[ci[7]];
   }
-  for (int k = j; k < len && k < j + D; ++k) a0 += (T)stream_load(v + k * kSlice) * xs[col(k)];
+  for (int k = j; k < len && k < j + D; ++k) a0 += (T)mat_load<NT>(v + k * kSlice) * xs[col(k)];
   return (a0 + a1) + (a2 + a3);
 }
 
@@ -231,7 +273,7 @@ __device__ __forceinline__ T sell_row_part(const MatArgs& A, const TV* __restric
 // wavefront takes chunks h, h + W, ... of four blocks.  A block adds to its
 // rows the dot of its row with the three x values of its node column; blocks
 // alternate between two partial sums per row, added at the end.
-template <typename T, typename TV = T>
+template <typename T, typename TV = T, bool NT = true>
 __device__ __forceinline__ void sell3_sum(const uint16_t* __restrict__ c16, const TV* __restrict__ v,
                                           const T* __restrict__ xs, int len, int h, int W, T (&acc)[3]) {
   constexpr int D = 4;
@@ -247,32 +289,35 @@ __device__ __forceinline__ void sell3_sum(const uint16_t* __restrict__ c16, cons
     int ci[D];
     TV vi[D][9];
 #pragma unroll
-    for (int u = 0; u < D; ++u) ci[u] = (int)stream_load(c16 + (j + u) * kSlice);
+    for (int u = 0; u < D; ++u) ci[u] = (int)mat_load<NT>(c16 + (j + u) * kSlice);
 #pragma unroll
     for (int u = 0; u < D; ++u)
 #pragma unroll
-      for (int t = 0; t < 9; ++t) vi[u][t] = stream_load(v + (size_t)(9 * (j + u) + t) * kSlice);
+      for (int t = 0; t < 9; ++t) vi[u][t] = mat_load<NT>(v + (size_t)(9 * (j + u) + t) * kSlice);
 #pragma unroll
     for (int u = 0; u < D; ++u) add(vi[u], ci[u], a[u & 1]);
   }
   for (int k = j; k < len && k < j + D; ++k) {
     TV vb[9];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) vb[t] = stream_load(v + (size_t)(9 * k + t) * kSlice);
-    add(vb, (int)stream_load(c16 + k * kSlice), a[(k - j) & 1]);
+    for (int t = 0; t < 9; ++t) vb[t] = mat_load<NT>(v + (size_t)(9 * k + t) * kSlice);
+    add(vb, (int)mat_load<NT>(c16 + k * kSlice), a[(k - j) & 1]);
   }
 #pragma unroll
   for (int r = 0; r < 3; ++r) acc[r] = a[0][r] + a[1][r];
 }
 
 // sell3_sum for lane `lane` of the slice whose blocks start at `base` (`len`
-// per node row, base node cb) of matrix A.
+// per node row, base node cb) of matrix A; `keep`: plain loads.
 template <typename T, typename TV = T>
 __device__ __forceinline__ void sell3_row_part(const MatArgs& A, const TV* __restrict__ vals,
-                                               const T* __restrict__ x, int base, int len, int cb, int lane, int h,
-                                               int W, T (&acc)[3]) {
-  sell3_sum<T, TV>(reinterpret_cast<const uint16_t*>(A.col) + base + lane, vals + (size_t)9 * base + lane,
-                   x + 3 * (size_t)cb, len, h, W, acc);
+                                               const T* __restrict__ x, bool keep, int base, int len, int cb,
+                                               int lane, int h, int W, T (&acc)[3]) {
+  const uint16_t* c16 = reinterpret_cast<const uint16_t*>(A.col) + base + lane;
+  const TV* v = vals + (size_t)9 * base + lane;
+  const T* xs = x + 3 * (size_t)cb;
+  if (keep) sell3_sum<T, TV, false>(c16, v, xs, len, h, W, acc);
+  else sell3_sum<T, TV, true>(c16, v, xs, len, h, W, acc);
 }
 
 // SELL3 form of for_each_row: f(row, (A x)_row) for the three rows 3k + c of
@@ -302,7 +347,8 @@ __device__ __forceinline__ void for_each_node_row(const MatArgs& A, const TV* __
       if (k < A.span) slot = ord[k];
       const int s = slot.x;
       T ax[3] = {(T)0, (T)0, (T)0};
-      if (s >= 0 && x) sell3_row_part<T, TV>(A, vals, x, slot.y, slot.z, slot.w, lane, W == 1 ? 0 : h, W, ax);
+      if (s >= 0 && x) 
+        sell3_row_part<T, TV>(A, vals, x, slice_kept<TV>(A, k), slot.y, slot.z, slot.w, lane, W == 1 ? 0 : h, W, ax);
       if (W == 1) {
         if (s >= 0) emit(s, ax);
         continue;
@@ -326,7 +372,8 @@ __device__ __forceinline__ void for_each_node_row(const MatArgs& A, const TV* __
       T ax[3] = {(T)0, (T)0, (T)0};
       if (x) {
         const int base = A.ptr[s];
-        sell3_row_part<T, TV>(A, vals, x, base, (A.ptr[s + 1] - base) / kSlice, A.cbase[s], lane, 0, 1, ax);
+        sell3_row_part<T, TV>(A, vals, x, slice_kept<TV>(A, s), base, (A.ptr[s + 1] - base) / kSlice, A.cbase[s],
+                              lane, 0, 1, ax);
       }
       emit(s, ax);
     }
@@ -344,10 +391,14 @@ __device__ __forceinline__ void for_each_row(const MatArgs& A, const TV* __restr
     auto one_slice = [&](int s) {
       T ax = (T)0;
       if (x) {
+        const bool keep = slice_kept<TV>(A, s);
+        const uint16_t* c16 = reinterpret_cast<const uint16_t*>(A.col);
         if constexpr (FMT == kFmtSell16)
-          ax = sell16_row<T, TV>(A.ptr, reinterpret_cast<const uint16_t*>(A.col), A.cbase, vals, x, s, lane);
+          ax = keep ? sell16_row<T, TV, false>(A.ptr, c16, A.cbase, vals, x, s, lane)
+                    : sell16_row<T, TV, true>(A.ptr, c16, A.cbase, vals, x, s, lane);
         else
-          ax = sell_row<T, TV>(A.ptr, A.col, vals, x, s, lane);
+          ax = keep ? sell_row<T, TV, false>(A.ptr, A.col, vals, x, s, lane)
+                    : sell_row<T, TV, true>(A.ptr, A.col, vals, x, s, lane);
       }
       const int row = s * kSlice + lane;
       if (row < A.n) f(row, ax);
@@ -366,6 +417,12 @@ __device__ __forceinline__ void for_each_row(const MatArgs& A, const TV* __restr
       const int xcd = blockIdx.x % kXcds, bpx = gridDim.x / kXcds;
       const int4* ord = reinterpret_cast<const int4*>(A.order) + (size_t)xcd * A.span;
       const int passes = (A.span + bpx * spb - 1) / (bpx * spb);
+      constexpr bool C16 = FMT == kFmtSell16;
+      auto part_sum = [&](const int4& slot, int k, int hh, int WW) -> T {
+        if (slice_kept<TV>(A, k))
+          return sell_row_part<T, C16, TV, false>(A, vals, x, slot.y, slot.z, slot.w, lane, hh, WW);
+        return sell_row_part<T, C16, TV, true>(A, vals, x, slot.y, slot.z, slot.w, lane, hh, WW);
+      };
       for (int ps = 0; ps < passes; ++ps) {
         const int k = (ps * bpx + blockIdx.x / kXcds) * spb + g;
         int4 slot = make_int4(-1, 0, 0, 0);
@@ -374,15 +431,14 @@ __device__ __forceinline__ void for_each_row(const MatArgs& A, const TV* __restr
         if (W == 1) {
           if (s >= 0) {
             T ax = (T)0;
-            if (x) ax = sell_row_part<T, FMT == kFmtSell16, TV>(A, vals, x, slot.y, slot.z, slot.w, lane, 0, 1);
+            if (x) ax = part_sum(slot, k, 0, 1);
             const int row = s * kSlice + lane;
             if (row < A.n) f(row, ax);
           }
           continue;
         }
         T ax = (T)0;
-        if (s >= 0 && x)
-          ax = sell_row_part<T, FMT == kFmtSell16, TV>(A, vals, x, slot.y, slot.z, slot.w, lane, h, W);
+        if (s >= 0 && x) ax = part_sum(slot, k, h, W);
         part[wave][lane] = ax;
         __syncthreads();
         if (h == 0 && s >= 0) {
