@@ -33,12 +33,37 @@ void set_error(const char* fmt, ...);
 
 constexpr int kWave = 64;
 
-// Wavefront sum (64 lanes) with DPP-free shuffles.
+// Wavefront sum (64 lanes), the result in every lane.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
   return v;
+}
+
+// A double from another lane of the same 16-lane row (DPP control CTRL).
+template <int CTRL>
+__device__ __forceinline__ double row_lane(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// The FP64 sum (64 active lanes), the same bits in every lane: pairs, quads, eights
+// and sixteens by DPP, the four row sums through scalar registers.  A reduction in
+// LDS shuffles is a chain of six round trips to the LDS, of which a solver's
+// iteration holds several.
+__device__ __forceinline__ double wave_sum(double v) {
+  v += row_lane<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += row_lane<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += row_lane<0x141>(v);  // row_half_mirror
+  v += row_lane<0x140>(v);  // row_mirror
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
 // Block-wide sum; `scratch` must hold blockDim.x/64 values. All threads get the result.

@@ -2,19 +2,21 @@
 // with FP64 residual replacement ("reliable updates"), and right-Jacobi
 // restarted GMRES (FP64).
 //
-// CG runs two fused kernels per iteration and keeps every scalar on the
-// device.  With q = A p maintained by the recurrence q = A z + beta q, the
-// search direction update folds into the SpMV kernel:
-//   K_A: p = z + beta p ; q = A z + beta q ; partial (p.q)
+// CG runs two launches per iteration and keeps every scalar on the device.  With
+// q = A p maintained by the recurrence q = A z + beta q, the search direction update
+// folds into the SpMV kernel:
+//   K_A: beta and the stopping tests from K_B's partials; p = z + beta p ;
+//        q = A z + beta q ; partial (p.q)
 //   K_B: alpha = rz / pq ; x += alpha p ; r -= alpha q ; z = D^-1 r ;
-//        partials (r.z), (r.r)                                -> beta (finisher)
-// Each bandwidth kernel leaves one partial sum per block.  K_B's blocks (few and
-// large, one round on the chip) each sum K_A's partials themselves in one fixed
-// order, so alpha needs no launch of its own; a one-block finisher reduces K_B's
-// partials (deterministic) and updates the device-side state for the next K_A.
-// No device-scope fence runs inside the bandwidth kernels, the host only looks
-// at the state every few iterations, and kernels return at once once the state
-// says stop.
+//        partials (r.z), (r.r)
+// Each bandwidth kernel leaves one partial sum per block, which every block of the
+// next kernel sums in one fixed order (the operands are loaded first and meet after
+// the block's own loads, so the sum costs no wait of its own).  Block 0 of K_A
+// records the iteration's scalars in the other of two state slots, so no block
+// reads what another block of its launch writes; a one-block finisher ends a chunk
+// of iterations.  No device-scope fence runs inside the bandwidth kernels, the host
+// only looks at the state every few iterations, and kernels return at once once the
+// state says stop.
 #include "mife_common.hpp"
 #include "mife_profile.hpp"
 #include "mife_sparse.hpp"
@@ -25,6 +27,7 @@ extern "C" int mife_profile_enable(int on);
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <vector>
 
@@ -38,14 +41,19 @@ constexpr int kFinThreads = 1024;  // one-block finishers: two partials per thre
 constexpr int kUpdateThreads = 1024;
 constexpr int kMaxIterChunk = 256;  // CG iterations launched between two host reads of the state
 
-struct CgState {
+struct CgScalars {
   double rz, pq, alpha, beta, rr, bb, tol2, scale;
   double rz_prev, maxrr, rr_seg, rr64;  // rr_seg: recurrence r.r when a segment ended
   // Segmented (mixed-precision) solves: a segment pauses once r.r <= seg_rr, set at
   // each replacement to seg_drop x the new r.r (seg_drop = 0: no pausing).
   double seg_drop, seg_rr;
   int iters, done, maxit, pause;
-  unsigned int cnt_a, cnt_b, cnt_c, pad2;
+};
+
+// Iteration k of a chunk reads s[k & 1] and leaves its scalars in s[(k + 1) & 1];
+// between chunks the state is s[0].
+struct CgState {
+  CgScalars s[2];
   // per-block partials of up to 4 reduced values each (value v of block b at v*kRedBlocks+b)
   double part_a[4 * kRedBlocks];
   double part_b[4 * kRedBlocks];
@@ -236,58 +244,157 @@ __global__ void fin_init_kernel(CgState* st, int nb, double tol2, int maxit) {
   double out[3];
   finish_sums<3>(st->part_b, nb, out);
   if (threadIdx.x == 0) {
-    st->rz = out[0];
-    st->rr = out[1];
-    st->bb = out[2];
-    st->maxrr = out[1];
-    st->beta = 0.0;
-    st->alpha = 0.0;
-    st->iters = 0;
-    st->maxit = maxit;
-    st->tol2 = tol2;
-    st->pause = 0;
-    st->done = (out[1] <= tol2 * out[2]) ? 1 : 0;
+    CgScalars& c = st->s[0];
+    c.rz = out[0];
+    c.rr = out[1];
+    c.bb = out[2];
+    c.maxrr = out[1];
+    c.beta = 0.0;
+    c.alpha = 0.0;
+    c.iters = 0;
+    c.maxit = maxit;
+    c.tol2 = tol2;
+    c.pause = 0;
+    c.done = (out[1] <= tol2 * out[2]) ? 1 : 0;
   }
 }
 
+__device__ __forceinline__ bool cg_done(const CgScalars& c, double rr) {
+  return rr <= c.tol2 * c.bb || c.iters + 1 >= c.maxit;
+}
+__device__ __forceinline__ bool cg_paused(const CgScalars& c, double rr) { return c.seg_rr > 0.0 && rr <= c.seg_rr; }
+
+// The scalars after an iteration's update: beta, the residual, the iteration count
+// and the stopping tests, from the update's sums r.z and r.r.
+__device__ __forceinline__ void cg_advance(CgScalars& c, double rz, double rr) {
+  c.done = cg_done(c, rr) ? 1 : 0;
+  c.pause = cg_paused(c, rr) ? 1 : 0;
+  c.rz_prev = c.rz;
+  c.beta = rz / c.rz;
+  c.rz = rz;
+  c.rr = rr;
+  c.iters += 1;
+  c.maxrr = fmax(c.maxrr, rr);
+}
+
+// Largest update grid: one block per CU, two partials per thread of a product block.
+constexpr int kUpdateGrid = 256;
+
+// A value that is the same in every lane, as a scalar.
+__device__ __forceinline__ double uniform(double v) {
+  const unsigned long long u = __double_as_longlong(v);
+  const unsigned int lo = __builtin_amdgcn_readfirstlane((int)(unsigned int)u);
+  const unsigned int hi = __builtin_amdgcn_readfirstlane((int)(unsigned int)(u >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Sums the update's nb (<= kUpdateGrid) partials of r.z and r.r in every block: the
+// loads are issued on construction, the sums meet around the row walk's first
+// barrier.  Without `pending` (a chunk's first iteration) the state stands.
+struct CgHook {
+  static constexpr bool kActive = true;
+  CgState* st;
+  double* red;
+  int k;
+  bool pending, stop;
+  double beta, v[2];
+  __device__ __forceinline__ CgHook(CgState* s, int kk, int nb, bool pend, double* r)
+      : st(s), red(r), k(kk), pending(pend), stop(false), beta(0.0) {
+    // wavefront w takes half w >> 1 of sum w & 1
+    const int i = 128 * (threadIdx.x >> 7) + (threadIdx.x & 63), j = threadIdx.x >> 6 & 1;
+    v[0] = pend && i < nb ? s->part_b[j * kRedBlocks + i] : 0.0;
+    v[1] = pend && i + 64 < nb ? s->part_b[j * kRedBlocks + i + 64] : 0.0;
+  }
+  __device__ __forceinline__ void stage() {
+    if (!pending) return;
+    const double s = wave_sum(v[0] + v[1]);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  }
+  __device__ __forceinline__ void finish() {
+    const CgScalars& in = st->s[k & 1];
+    if (!pending) {
+      beta = in.beta;
+      if (blockIdx.x == 0 && threadIdx.x == 0) st->s[(k + 1) & 1] = in;
+      return;
+    }
+    const double rz = uniform(red[0] + red[2]), rr = uniform(red[1] + red[3]);
+    beta = rz / in.rz;
+    stop = cg_done(in, rr) || cg_paused(in, rr);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      CgScalars c = in;
+      cg_advance(c, rz, rr);
+      st->s[(k + 1) & 1] = c;
+    }
+  }
+};
+
+template <typename T>
+struct CgRow {
+  T z, p, q;
+};
+
+// The product is formed before the previous iteration's sums are known: it depends
+// on z alone, beta enters with the row's p and q.  When those sums end the solve (or
+// pause it) the rows are left as they are.  Measured, against a one-block finisher
+// between update and product: FP64 CG on 96x32x32 elasticity 62.3 -> 57.4 ms (1,309
+// iterations), on a 16^3 trilinear system 13.2 -> 9.9 us per iteration; the mixed
+// 48^3 triquadratic pass 37.4 -> 37.3 ms (each of its 12 segments ends in a product
+// that is not used).
 template <typename T, int FMT, int L>
 __global__ __launch_bounds__(256) void cg_spmv_kernel(MatArgs A, const T* __restrict__ vals,
                                                       const T* __restrict__ z, T* __restrict__ p,
-                                                      T* __restrict__ q, CgState* st) {
-  if (st->done || st->pause) return;
-  const T beta = (T)st->beta;
+                                                      T* __restrict__ q, CgState* st, int k, int nb, int pending) {
+  __shared__ double red[4];
+  const CgScalars& in = st->s[k & 1];
+  if (in.done || in.pause) {  // carried forward so that every later launch sees it
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->s[(k + 1) & 1] = in;
+    return;
+  }
+  CgHook hook(st, k, nb, pending != 0, red);
   double m[1] = {0.0};
-  for_each_row<T, FMT, L>(A, vals, z, [&](int row, T az) {
-    const T pi = z[row] + beta * p[row];
-    const T qi = az + beta * q[row];
-    p[row] = pi;
-    q[row] = qi;
-    m[0] += (double)pi * (double)qi;
-  });
+  walk_rows<T, FMT, L>(
+      A, vals, z, [&](int row) { return CgRow<T>{z[row], p[row], q[row]}; },
+      [&](int row, T az, const CgRow<T>& w) {
+        if (hook.stop) return;
+        const T beta = (T)hook.beta;
+        const T pi = w.z + beta * w.p;
+        const T qi = az + beta * w.q;
+        p[row] = pi;
+        q[row] = qi;
+        m[0] += (double)pi * (double)qi;
+      },
+      hook);
   block_partials<1>(m, st->part_a);
 }
 
 // alpha = rz / (p.q) from K_A's nb_a partials (summed in every block), then
-// x += alpha p, r -= alpha q, z = D^-1 r and the r.z, r.r partials.  Block 0
-// records pq and alpha, which no block of this kernel reads.  Each thread takes
-// R = 16 / sizeof(T) consecutive rows through 16-byte vector accesses (R = 1
-// when a vector is not 16-byte aligned); rows past the last full group are
-// taken one per thread.
+// x += alpha p, r -= alpha q, z = D^-1 r and the r.z, r.r partials.  Each thread
+// takes R = 16 / sizeof(T) consecutive rows through 16-byte vector accesses (R = 1
+// when a vector is not 16-byte aligned), its first group's loads issued before the
+// partials are summed; rows past the last full group are taken one per thread.
 template <typename T, int R>
 __global__ __launch_bounds__(kUpdateThreads) void cg_update_kernel(int n, int nb_a, T* __restrict__ x,
                                                                    T* __restrict__ r, T* __restrict__ z,
                                                                    const T* __restrict__ p,
                                                                    const T* __restrict__ q,
-                                                                   const T* __restrict__ dinv, CgState* st) {
-  if (st->done || st->pause) return;
+                                                                   const T* __restrict__ dinv, CgState* st, int k) {
+  const CgScalars& c = st->s[(k + 1) & 1];
+  if (c.done || c.pause) return;
+  typedef T VT __attribute__((ext_vector_type(R)));
+  const int nv = n / R;
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x, nth = gridDim.x * blockDim.x;
+  VT xv{}, rv{}, pv{}, qv{}, dv{};
+  auto load = [&](int v) {
+    xv = reinterpret_cast<VT*>(x)[v];
+    rv = reinterpret_cast<VT*>(r)[v];
+    pv = reinterpret_cast<const VT*>(p)[v];
+    qv = reinterpret_cast<const VT*>(q)[v];
+    dv = reinterpret_cast<const VT*>(dinv)[v];
+  };
+  if (tid < nv) load(tid);
   double pq[1];
   finish_sums<1>(st->part_a, nb_a, pq);
-  const double alpha64 = st->rz / pq[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st->pq = pq[0];
-    st->alpha = alpha64;
-  }
-  const T alpha = (T)alpha64;
+  const T alpha = (T)(c.rz / pq[0]);
   double m[2] = {0.0, 0.0};
   auto row = [&](T& xi, T& ri, T& zi, T pi, T qi, T di) {
     xi += alpha * pi;
@@ -296,28 +403,22 @@ __global__ __launch_bounds__(kUpdateThreads) void cg_update_kernel(int n, int nb
     m[0] += (double)ri * (double)zi;
     m[1] += (double)ri * (double)ri;
   };
-  const int nv = n / R;
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x, nth = gridDim.x * blockDim.x;
-  if constexpr (R > 1) {
-    typedef T VT __attribute__((ext_vector_type(R)));
-    for (int v = tid; v < nv; v += nth) {
-      VT xv = reinterpret_cast<VT*>(x)[v], rv = reinterpret_cast<VT*>(r)[v], zv;
-      const VT pv = reinterpret_cast<const VT*>(p)[v], qv = reinterpret_cast<const VT*>(q)[v];
-      const VT dv = reinterpret_cast<const VT*>(dinv)[v];
+  for (int v = tid; v < nv; v += nth) {
+    if (v != tid) load(v);
+    VT zv;
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
-        T xi = xv[j], ri = rv[j], zi;
-        row(xi, ri, zi, pv[j], qv[j], dv[j]);
-        xv[j] = xi;
-        rv[j] = ri;
-        zv[j] = zi;
-      }
-      reinterpret_cast<VT*>(x)[v] = xv;
-      reinterpret_cast<VT*>(r)[v] = rv;
-      reinterpret_cast<VT*>(z)[v] = zv;
+    for (int j = 0; j < R; ++j) {
+      T xi = xv[j], ri = rv[j], zi;
+      row(xi, ri, zi, pv[j], qv[j], dv[j]);
+      xv[j] = xi;
+      rv[j] = ri;
+      zv[j] = zi;
     }
+    reinterpret_cast<VT*>(x)[v] = xv;
+    reinterpret_cast<VT*>(r)[v] = rv;
+    reinterpret_cast<VT*>(z)[v] = zv;
   }
-  for (int i = (R > 1 ? nv * R : 0) + tid; i < n; i += nth) {
+  for (int i = nv * R + tid; i < n; i += nth) {
     T xi = x[i], ri = r[i], zi;
     row(xi, ri, zi, p[i], q[i], dinv[i]);
     x[i] = xi;
@@ -327,19 +428,15 @@ __global__ __launch_bounds__(kUpdateThreads) void cg_update_kernel(int n, int nb
   block_partials<2>(m, st->part_b);
 }
 
-__global__ void fin_beta_kernel(CgState* st, int nb) {
-  if (st->done || st->pause) return;
+// End of a chunk of `count` iterations: the last one's scalars (unless the state
+// already says stop), left in s[0].
+__global__ void fin_beta_kernel(CgState* st, int count, int nb) {
   double out[2];
   finish_sums<2>(st->part_b, nb, out);
   if (threadIdx.x == 0) {
-    st->rz_prev = st->rz;
-    st->beta = out[0] / st->rz;
-    st->rz = out[0];
-    st->rr = out[1];
-    st->iters += 1;
-    st->maxrr = fmax(st->maxrr, out[1]);
-    st->done = (out[1] <= st->tol2 * st->bb || st->iters >= st->maxit) ? 1 : 0;
-    st->pause = (st->seg_rr > 0.0 && out[1] <= st->seg_rr) ? 1 : 0;
+    CgScalars c = st->s[count & 1];
+    if (!c.done && !c.pause) cg_advance(c, out[0], out[1]);
+    st->s[0] = c;
   }
 }
 
@@ -363,10 +460,11 @@ __global__ void fin_residual_kernel(CgState* st, int nb) {
   double out[2];
   finish_sums<2>(st->part_a, nb, out);
   if (threadIdx.x == 0) {
-    st->rr64 = out[0];
-    st->rr = out[0];
-    st->bb = out[1];
-    st->scale = sqrt(out[0]);
+    CgScalars& c = st->s[0];
+    c.rr64 = out[0];
+    c.rr = out[0];
+    c.bb = out[1];
+    c.scale = sqrt(out[0]);
   }
 }
 
@@ -433,18 +531,20 @@ __global__ void fin_replace_kernel(CgState* st, const CgState* ro, int nb, int f
   double out[2];
   finish_sums<2>(st->part_b, nb, out);
   if (threadIdx.x == 0) {
-    st->rr_seg = st->rr;
-    st->rr64 = ro->rr64;
-    st->beta = (first || out[1] > kRestartGrowth * st->rr) ? 0.0 : out[0] / st->rz_prev;
-    st->rz = out[0];
-    st->rr = out[1];
-    st->maxrr = out[1];
-    st->bb = ro->bb;
-    st->pause = 0;
+    CgScalars& c = st->s[0];
+    const CgScalars& t = ro->s[0];
+    c.rr_seg = c.rr;
+    c.rr64 = t.rr64;
+    c.beta = (first || out[1] > kRestartGrowth * c.rr) ? 0.0 : out[0] / c.rz_prev;
+    c.rz = out[0];
+    c.rr = out[1];
+    c.maxrr = out[1];
+    c.bb = t.bb;
+    c.pause = 0;
     // the next segment ends when the recurrence has fallen by seg_drop, or at a
     // quarter of the target r.r when that is nearer
-    st->seg_rr = st->seg_drop > 0.0 ? fmax(st->seg_drop * out[1], 0.25 * tol2 * ro->bb) : 0.0;
-    st->done = (ro->rr64 <= tol2 * ro->bb) ? 1 : 0;
+    c.seg_rr = c.seg_drop > 0.0 ? fmax(c.seg_drop * out[1], 0.25 * tol2 * t.bb) : 0.0;
+    c.done = (t.rr64 <= tol2 * t.bb) ? 1 : 0;
   }
 }
 
@@ -903,27 +1003,42 @@ static void launch_cg_init(const Mat& M, const T* vals, const T* b, const T* x, 
   prof::end(tk, s, prof::kCgInit);
 }
 
-// Launches one CG iteration (SpMV kernel, update kernel, finisher); with
-// profiling on, the two bandwidth kernels' event tickets are returned through
-// tk[0..1] (else -1).
+// Grid of the update kernel (its partials are summed by every product block).
+static bool update_vectorised(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if (!aligned16(p)) return false;
+  return true;
+}
+
+static int update_grid(int n, int R) { return std::max(1, std::min(div_up(div_up(n, R), kUpdateThreads), kUpdateGrid)); }
+
+// Launches iteration k of a chunk (SpMV kernel, update kernel); with profiling on,
+// the two kernels' event tickets are returned through tk[0..1] (else -1).
 template <typename T>
 static void launch_cg_iter(const Mat& M, const T* vals, T* x, T* r, T* z, T* p, T* q, const T* dinv, CgState* st,
-                           hipStream_t s, int* tk) {
+                           int k, hipStream_t s, int* tk) {
   const int grid = row_grid(M.a, M.a.fmt != MIFE_FMT_CSR ? 64 : M.L);
   constexpr int R = 16 / sizeof(T);
-  const bool vec = aligned16(x) && aligned16(r) && aligned16(z) && aligned16(p) && aligned16(q) && aligned16(dinv);
-  const int units = vec ? div_up(M.a.n, R) : M.a.n;
-  const int ug = std::max(1, std::min(div_up(units, kUpdateThreads), kMaxGrid));
+  const bool vec = update_vectorised({x, r, z, p, q, dinv});
+  const int ug = update_grid(M.a.n, vec ? R : 1);
   tk[0] = prof::begin(s);
-  MIFE_DISPATCH_FMT(M.a, M.L, (cg_spmv_kernel<T, FMT_, L_><<<grid, 256, 0, s>>>(M.a, vals, z, p, q, st)));
+  MIFE_DISPATCH_FMT(M.a, M.L, (cg_spmv_kernel<T, FMT_, L_><<<grid, 256, 0, s>>>(M.a, vals, z, p, q, st, k, ug,
+                                                                                  k > 0 ? 1 : 0)));
   prof::end(tk[0], s, sizeof(T) == 8 ? prof::kCgSpmv : prof::kCgSpmv32);
   tk[1] = prof::begin(s);
   if (vec)
-    cg_update_kernel<T, R><<<ug, kUpdateThreads, 0, s>>>(M.a.n, grid, x, r, z, p, q, dinv, st);
+    cg_update_kernel<T, R><<<ug, kUpdateThreads, 0, s>>>(M.a.n, grid, x, r, z, p, q, dinv, st, k);
   else
-    cg_update_kernel<T, 1><<<ug, kUpdateThreads, 0, s>>>(M.a.n, grid, x, r, z, p, q, dinv, st);
+    cg_update_kernel<T, 1><<<ug, kUpdateThreads, 0, s>>>(M.a.n, grid, x, r, z, p, q, dinv, st, k);
   prof::end(tk[1], s, sizeof(T) == 8 ? prof::kCgUpdate : prof::kCgUpdate32);
-  fin_beta_kernel<<<1, kFinThreads, 0, s>>>(st, ug);
+}
+
+// The finisher of a chunk of `count` iterations.
+template <typename T>
+static void launch_cg_finish(const Mat& M, const T* x, const T* r, const T* z, const T* p, const T* q, const T* dinv,
+                             CgState* st, int count, hipStream_t s) {
+  const bool vec = update_vectorised({x, r, z, p, q, dinv});
+  fin_beta_kernel<<<1, kFinThreads, 0, s>>>(st, count, update_grid(M.a.n, vec ? 16 / (int)sizeof(T) : 1));
 }
 
 template <typename TV = double>
@@ -937,15 +1052,10 @@ static void launch_residual64(const Mat& M, const TV* vals, const double* b, con
   fin_residual_kernel<<<1, kFinThreads, 0, s>>>(st, grid);
 }
 
-struct HostState {
-  double rz, pq, alpha, beta, rr, bb, tol2, scale;
-  double rz_prev, maxrr, rr_seg, rr64;
-  double seg_drop, seg_rr;
-  int iters, done, maxit, pause;
-};
+using HostState = CgScalars;
 
 static int read_state(const CgState* st, HostState* h, hipStream_t s) {
-  MIFE_CHECK_HIP(hipMemcpyAsync(h, st, sizeof(HostState), hipMemcpyDeviceToHost, s));
+  MIFE_CHECK_HIP(hipMemcpyAsync(h, &st->s[0], sizeof(HostState), hipMemcpyDeviceToHost, s));
   MIFE_CHECK_HIP(hipStreamSynchronize(s));
   return MIFE_OK;
 }
@@ -1009,7 +1119,8 @@ static int cg_chunk_graph(const Mat& M, const T* vals, T* x, T* r, T* z, T* p, T
   if (!cs) MIFE_CHECK_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
   MIFE_CHECK_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
   int tk[2];
-  for (int k = 0; k < kGraphIters; ++k) launch_cg_iter<T>(M, vals, x, r, z, p, q, dinv, st, cs, tk);
+  for (int k = 0; k < kGraphIters; ++k) launch_cg_iter<T>(M, vals, x, r, z, p, q, dinv, st, k, cs, tk);
+  launch_cg_finish<T>(M, x, r, z, p, q, dinv, st, kGraphIters, cs);
   hipGraph_t graph = nullptr;
   const hipError_t ce = hipStreamEndCapture(cs, &graph);
   MIFE_REQUIRE(ce == hipSuccess && graph, MIFE_ERR_HIP, "CG chunk capture failed: %s", hipGetErrorString(ce));
@@ -1028,7 +1139,7 @@ static int cg_chunk_graph(const Mat& M, const T* vals, T* x, T* r, T* z, T* p, T
   return MIFE_OK;
 }
 
-// Launches exactly `count` (<= kMaxIterChunk) CG iterations after iteration it0
+// Launches exactly `count` (1 .. kMaxIterChunk) CG iterations after iteration it0
 // (iterations after a device-side stop return at once), no synchronisation.
 // Small systems with profiling off replay the cached graph of kGraphIters
 // iterations count / kGraphIters times and launch the rest one by one (the
@@ -1044,8 +1155,9 @@ static int launch_iters(const Mat& M, const T* vals, T* x, T* r, T* z, T* p, T* 
     int rc = cg_chunk_graph<T>(M, vals, x, r, z, p, q, dinv, st, &exec);
     if (rc) return rc;
     for (int c = 0; c < count / kGraphIters; ++c) MIFE_CHECK_HIP(hipGraphLaunch(exec, s));
-    for (int k = count / kGraphIters * kGraphIters; k < count; ++k)
-      launch_cg_iter<T>(M, vals, x, r, z, p, q, dinv, st, s, &tickets[2 * k]);
+    const int rest = count % kGraphIters;
+    for (int k = 0; k < rest; ++k) launch_cg_iter<T>(M, vals, x, r, z, p, q, dinv, st, k, s, &tickets[2 * k]);
+    if (rest) launch_cg_finish<T>(M, x, r, z, p, q, dinv, st, rest, s);
     for (int k = 0; k < 2 * count; ++k) tickets[k] = -1;
     MIFE_CHECK_HIP(hipGetLastError());
     return MIFE_OK;
@@ -1053,9 +1165,10 @@ static int launch_iters(const Mat& M, const T* vals, T* x, T* r, T* z, T* p, T* 
   for (int k = 0; k < count; ++k) {
     const bool sample = on && ((it0 + k) % 8) == 0;
     if (on && !sample) mife_profile_enable(0);
-    launch_cg_iter<T>(M, vals, x, r, z, p, q, dinv, st, s, &tickets[2 * k]);
+    launch_cg_iter<T>(M, vals, x, r, z, p, q, dinv, st, k, s, &tickets[2 * k]);
     if (on && !sample) mife_profile_enable(1);
   }
+  launch_cg_finish<T>(M, x, r, z, p, q, dinv, st, count, s);
   MIFE_CHECK_HIP(hipGetLastError());
   return MIFE_OK;
 }
@@ -1418,7 +1531,7 @@ int mife_refine(const mife_matrix* A, const double* vals64, const float* vals32,
   init.maxit = maxit;
   init.seg_drop = delta2;
   const double tol2 = rtol * rtol;
-  MIFE_CHECK_HIP(hipMemcpyAsync(st, &init, sizeof(HostState), hipMemcpyHostToDevice, s));
+  MIFE_CHECK_HIP(hipMemcpyAsync(&st->s[0], &init, sizeof(HostState), hipMemcpyHostToDevice, s));
   HostState hs{};
   int nrep = 0;
   bool first = true;

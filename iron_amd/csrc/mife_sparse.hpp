@@ -320,22 +320,57 @@ __device__ __forceinline__ void sell3_row_part(const MatArgs& A, const TV* __res
   else sell3_sum<T, TV, true>(c16, v, xs, len, h, W, acc);
 }
 
-// SELL3 form of for_each_row: f(row, (A x)_row) for the three rows 3k + c of
+// What a row walk does besides the rows.  pre(row) runs before the row's sum, on
+// the lane that will emit the row, and its result is handed to f: loads it issues
+// are in flight during the product.  hook.stage() and hook.finish() run once per
+// block around the walk's first barrier, after the block's first product (walks
+// without a schedule: before their rows): a block-wide sum whose operands were
+// loaded at the start of the kernel is formed there without a barrier or a wait of
+// its own.
+// Blocks of a row walk have kWalkWaves wavefronts.
+constexpr int kWalkWaves = 4;
+
+struct NoPre {
+  __device__ __forceinline__ int operator()(int) const { return 0; }
+};
+struct NoHook {
+  static constexpr bool kActive = false;
+  __device__ __forceinline__ void stage() {}
+  __device__ __forceinline__ void finish() {}
+};
+
+template <typename H>
+__device__ __forceinline__ void hook_now(H& hook) {
+  if constexpr (H::kActive) {
+    hook.stage();
+    __syncthreads();
+    hook.finish();
+  }
+}
+
+// SELL3 form of walk_rows: f(row, (A x)_row, pre(row)) for the three rows 3k + c of
 // each node row k.
-template <typename T, typename TV, typename F>
-__device__ __forceinline__ void for_each_node_row(const MatArgs& A, const TV* __restrict__ vals,
-                                                  const T* __restrict__ x, F&& f) {
+template <typename T, typename TV, typename P, typename F, typename H>
+__device__ __forceinline__ void walk_node_rows(const MatArgs& A, const TV* __restrict__ vals,
+                                               const T* __restrict__ x, P&& pre, F&& f, H& hook) {
+  using PV = decltype(pre(0));
   const int wpb = blockDim.x >> 6, lane = threadIdx.x & 63;
-  auto emit = [&](int s, const T (&ax)[3]) {
+  auto prepare = [&](int s, bool own, PV (&pv)[3]) {
     const int row = 3 * (s * kSlice + lane);
 #pragma unroll
     for (int c = 0; c < 3; ++c)
-      if (row + c < A.n) f(row + c, ax[c]);
+      if (own && row + c < A.n) pv[c] = pre(row + c);
+  };
+  auto emit = [&](int s, const T (&ax)[3], const PV (&pv)[3]) {
+    const int row = 3 * (s * kSlice + lane);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      if (row + c < A.n) f(row + c, ax[c], pv[c]);
   };
   if (A.order) {
     // scheduled, as the scalar SELL path: W wavefronts share a slice and their
     // partial sums meet in LDS, added in a fixed order by the first of them
-    __shared__ T part[3][16][kSlice];
+    __shared__ T part[3][kWalkWaves][kSlice];
     const int W = min(A.split, wpb), spb = wpb / W;
     const int wave = threadIdx.x >> 6, g = wave / W, h = wave - g * W;
     const int xcd = blockIdx.x % kXcds, bpx = gridDim.x / kXcds;
@@ -346,50 +381,57 @@ __device__ __forceinline__ void for_each_node_row(const MatArgs& A, const TV* __
       int4 slot = make_int4(-1, 0, 0, 0);
       if (k < A.span) slot = ord[k];
       const int s = slot.x;
+      const bool own = s >= 0 && h == 0;
+      PV pv[3] = {};
+      prepare(s, own, pv);
       T ax[3] = {(T)0, (T)0, (T)0};
-      if (s >= 0 && x) 
-        sell3_row_part<T, TV>(A, vals, x, slice_kept<TV>(A, k), slot.y, slot.z, slot.w, lane, W == 1 ? 0 : h, W, ax);
-      if (W == 1) {
-        if (s >= 0) emit(s, ax);
-        continue;
-      }
+      if (s >= 0 && x)
+        sell3_row_part<T, TV>(A, vals, x, slice_kept<TV>(A, k), slot.y, slot.z, slot.w, lane, h, W, ax);
+      if (W > 1) {
 #pragma unroll
-      for (int c = 0; c < 3; ++c) part[c][wave][lane] = ax[c];
-      __syncthreads();
-      if (h == 0 && s >= 0) {
-        T t[3];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          t[c] = part[c][wave][lane];
-          for (int q = 1; q < W; ++q) t[c] += part[c][wave + q][lane];
-        }
-        emit(s, t);
+        for (int c = 0; c < 3; ++c) part[c][wave][lane] = ax[c];
       }
-      __syncthreads();
+      if (ps == 0) hook.stage();
+      if (W > 1 || (H::kActive && ps == 0)) __syncthreads();
+      if (ps == 0 && h == 0) hook.finish();
+      if (own) {
+        for (int q = 1; q < W; ++q)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) ax[c] += part[c][wave + q][lane];
+        emit(s, ax, pv);
+      }
+      if (W > 1 && ps + 1 < passes) __syncthreads();
     }
   } else {
+    hook_now(hook);
     for (int s = blockIdx.x * wpb + (threadIdx.x >> 6); s < A.n_slices; s += gridDim.x * wpb) {
+      PV pv[3] = {};
+      prepare(s, true, pv);
       T ax[3] = {(T)0, (T)0, (T)0};
       if (x) {
         const int base = A.ptr[s];
         sell3_row_part<T, TV>(A, vals, x, slice_kept<TV>(A, s), base, (A.ptr[s + 1] - base) / kSlice, A.cbase[s],
                               lane, 0, 1, ax);
       }
-      emit(s, ax);
+      emit(s, ax, pv);
     }
   }
 }
 
-// Calls f(row, (A x)_row) once per row (by one lane), over the whole grid.
-template <typename T, int FMT, int L, typename TV = T, typename F>
-__device__ __forceinline__ void for_each_row(const MatArgs& A, const TV* __restrict__ vals, const T* __restrict__ x,
-                                             F&& f) {
+// Calls f(row, (A x)_row, pre(row)) once per row (by one lane), over the whole grid.
+template <typename T, int FMT, int L, typename TV = T, typename P, typename F, typename H>
+__device__ __forceinline__ void walk_rows(const MatArgs& A, const TV* __restrict__ vals, const T* __restrict__ x,
+                                          P&& pre, F&& f, H& hook) {
+  using PV = decltype(pre(0));
   if constexpr (FMT == kFmtSell3) {
-    for_each_node_row<T, TV>(A, vals, x, f);
+    walk_node_rows<T, TV>(A, vals, x, pre, f, hook);
   } else if constexpr (FMT == MIFE_FMT_SELL || FMT == kFmtSell16) {
     const int wpb = blockDim.x >> 6, lane = threadIdx.x & 63;
     auto one_slice = [&](int s) {
       T ax = (T)0;
+      const int row = s * kSlice + lane;
+      PV pv{};
+      if (row < A.n) pv = pre(row);
       if (x) {
         const bool keep = slice_kept<TV>(A, s);
         const uint16_t* c16 = reinterpret_cast<const uint16_t*>(A.col);
@@ -400,8 +442,7 @@ __device__ __forceinline__ void for_each_row(const MatArgs& A, const TV* __restr
           ax = keep ? sell_row<T, TV, false>(A.ptr, A.col, vals, x, s, lane)
                     : sell_row<T, TV, true>(A.ptr, A.col, vals, x, s, lane);
       }
-      const int row = s * kSlice + lane;
-      if (row < A.n) f(row, ax);
+      if (row < A.n) f(row, ax, pv);
     };
     if (A.order) {
       // Scheduled: the dispatcher places block b on XCD b % 8, which walks its own
@@ -411,55 +452,61 @@ __device__ __forceinline__ void for_each_row(const MatArgs& A, const TV* __restr
       // wavefront); their partial row sums meet in LDS and the first of them adds
       // them in a fixed order.  Every wavefront of a block makes the same number of
       // passes, so the barriers are uniform.
-      __shared__ T part[16][kSlice];
+      __shared__ T part[kWalkWaves][kSlice];
       const int W = min(A.split, wpb), spb = wpb / W;
       const int wave = threadIdx.x >> 6, g = wave / W, h = wave - g * W;
       const int xcd = blockIdx.x % kXcds, bpx = gridDim.x / kXcds;
       const int4* ord = reinterpret_cast<const int4*>(A.order) + (size_t)xcd * A.span;
       const int passes = (A.span + bpx * spb - 1) / (bpx * spb);
       constexpr bool C16 = FMT == kFmtSell16;
-      auto part_sum = [&](const int4& slot, int k, int hh, int WW) -> T {
-        if (slice_kept<TV>(A, k))
-          return sell_row_part<T, C16, TV, false>(A, vals, x, slot.y, slot.z, slot.w, lane, hh, WW);
-        return sell_row_part<T, C16, TV, true>(A, vals, x, slot.y, slot.z, slot.w, lane, hh, WW);
-      };
       for (int ps = 0; ps < passes; ++ps) {
         const int k = (ps * bpx + blockIdx.x / kXcds) * spb + g;
         int4 slot = make_int4(-1, 0, 0, 0);
         if (k < A.span) slot = ord[k];
-        const int s = slot.x;
-        if (W == 1) {
-          if (s >= 0) {
-            T ax = (T)0;
-            if (x) ax = part_sum(slot, k, 0, 1);
-            const int row = s * kSlice + lane;
-            if (row < A.n) f(row, ax);
-          }
-          continue;
-        }
+        const int s = slot.x, row = s * kSlice + lane;
+        const bool own = s >= 0 && h == 0 && row < A.n;
+        PV pv{};
+        if (own) pv = pre(row);
         T ax = (T)0;
-        if (s >= 0 && x) ax = part_sum(slot, k, h, W);
-        part[wave][lane] = ax;
-        __syncthreads();
-        if (h == 0 && s >= 0) {
-          T t = part[wave][lane];
-          for (int q = 1; q < W; ++q) t += part[wave + q][lane];
-          const int row = s * kSlice + lane;
-          if (row < A.n) f(row, t);
+        if (s >= 0 && x) {
+          if (slice_kept<TV>(A, k))
+            ax = sell_row_part<T, C16, TV, false>(A, vals, x, slot.y, slot.z, slot.w, lane, h, W);
+          else
+            ax = sell_row_part<T, C16, TV, true>(A, vals, x, slot.y, slot.z, slot.w, lane, h, W);
         }
-        __syncthreads();
+        if (W > 1) part[wave][lane] = ax;
+        if (ps == 0) hook.stage();
+        if (W > 1 || (H::kActive && ps == 0)) __syncthreads();
+        if (ps == 0 && h == 0) hook.finish();
+        if (own) {
+          for (int q = 1; q < W; ++q) ax += part[wave + q][lane];
+          f(row, ax, pv);
+        }
+        if (W > 1 && ps + 1 < passes) __syncthreads();
       }
     } else {
+      hook_now(hook);
       for (int s = blockIdx.x * wpb + (threadIdx.x >> 6); s < A.n_slices; s += gridDim.x * wpb) one_slice(s);
     }
   } else {
+    hook_now(hook);
     const int gpb = blockDim.x / L, sub = threadIdx.x % L;
     for (int row = blockIdx.x * gpb + threadIdx.x / L; row < A.n; row += gridDim.x * gpb) {
+      PV pv{};
+      if (sub == 0) pv = pre(row);
       T ax = 0;
       if (x) ax = group_sum<T, L>(row_partial<T, L, TV>(A.ptr, A.col, vals, x, row, sub));
-      if (sub == 0) f(row, ax);
+      if (sub == 0) f(row, ax, pv);
     }
   }
+}
+
+// Calls f(row, (A x)_row) once per row (by one lane), over the whole grid.
+template <typename T, int FMT, int L, typename TV = T, typename F>
+__device__ __forceinline__ void for_each_row(const MatArgs& A, const TV* __restrict__ vals, const T* __restrict__ x,
+                                             F&& f) {
+  NoHook none;
+  walk_rows<T, FMT, L, TV>(A, vals, x, NoPre{}, [&](int row, T ax, int) { f(row, ax); }, none);
 }
 
 // Lanes per CSR row from the mean row length.
