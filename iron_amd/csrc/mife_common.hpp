@@ -54,15 +54,23 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
                           __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
+// Sums over aligned groups of 8 or 16 lanes, the same bits in every lane of a group.
+__device__ __forceinline__ double sum8(double v) {
+  v += row_lane<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += row_lane<0x4E>(v);   // quad_perm [2,3,0,1]
+  return v + row_lane<0x141>(v);  // row_half_mirror
+}
+__device__ __forceinline__ double sum16(double v) {
+  v = sum8(v);
+  return v + row_lane<0x140>(v);  // row_mirror
+}
+
 // The FP64 sum (64 active lanes), the same bits in every lane: pairs, quads, eights
 // and sixteens by DPP, the four row sums through scalar registers.  A reduction in
 // LDS shuffles is a chain of six round trips to the LDS, of which a solver's
 // iteration holds several.
 __device__ __forceinline__ double wave_sum(double v) {
-  v += row_lane<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += row_lane<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += row_lane<0x141>(v);  // row_half_mirror
-  v += row_lane<0x140>(v);  // row_mirror
+  v = sum16(v);
   return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 

@@ -71,47 +71,80 @@ __global__ void sell_build_kernel(int n, const int32_t* __restrict__ rp, const i
   }
 }
 
-// One wavefront per free row: b[f] = src + rhs - sum over fixed columns of K_ij u_j,
-// skipping |u_j| < ZT or |K_ij| < ZT as SOLVER_MATRICES_STATIC_ASSEMBLE does.
-// 64 free rows per wavefront, one per lane: each lane forms src + rhs of its row;
-// then the wavefront walks the rows that take a lifting term (a ballot of the
-// lanes), all 64 lanes over each such row's entries.  The sums are those of one
-// wavefront per row, in the same order.
-__global__ void solver_rhs_kernel(int n_free, const int32_t* __restrict__ free_idx,
-                                  const int32_t* __restrict__ row_ptr, const int32_t* __restrict__ col,
-                                  const double* __restrict__ vals, const int32_t* __restrict__ new_idx,
-                                  const double* __restrict__ u, const double* __restrict__ src,
-                                  const double* __restrict__ rhs, const uint8_t* __restrict__ rhs_fixed,
-                                  double* __restrict__ b) {
+// b[f] = src + rhs - sum over fixed columns of K_ij u_j, skipping |u_j| < ZT or
+// |K_ij| < ZT as SOLVER_MATRICES_STATIC_ASSEMBLE does.  Bound by latency: every row
+// waits for DOF -> flag, source and bounds, and the rows near the boundary for
+// column -> DOF number -> values.  So a block takes four runs of 64 free rows, far
+// apart so that a boundary plane's rows spread over many blocks; each wavefront forms
+// src + rhs of one run, one row per lane, and lists the rows that take a lifting
+// term; then 16 lanes walk each listed row, 16 rows side by side, four entries in
+// flight per lane.  75 x 83 x 67 nodes, source and every face fixed: 197 us with
+// the listed rows of 64 walked by one wavefront one by one, 75 us with each fixed
+// entry's loads behind its own test, 38 us now.
+constexpr int kRhsRows = 256;
+
+__global__ __launch_bounds__(256) void solver_rhs_kernel(int n_free, const int32_t* __restrict__ free_idx,
+                                                         const int32_t* __restrict__ row_ptr,
+                                                         const int32_t* __restrict__ col,
+                                                         const double* __restrict__ vals,
+                                                         const int32_t* __restrict__ new_idx,
+                                                         const double* __restrict__ u, const double* __restrict__ src,
+                                                         const double* __restrict__ rhs,
+                                                         const uint8_t* __restrict__ rhs_fixed,
+                                                         double* __restrict__ b) {
+  __shared__ int k0s[kRhsRows], k1s[kRhsRows], who[kRhsRows], count;
+  __shared__ double lift_s[kRhsRows];
   const double ZT = 5.0 * 2.220446049250313e-16;
-  const int lane = threadIdx.x & 63;
-  const int f = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64 + lane;
-  int i = -1;
-  double v = 0.0, mine = 0.0;
-  bool need = false;
-  if (f < n_free) {
-    i = free_idx[f];
+  const int t = threadIdx.x, sub = t & 15;
+  const long long f = ((long long)(t >> 6) * gridDim.x + blockIdx.x) * 64 + (t & 63);
+  const bool own = f < n_free;
+  if (t == 0) count = 0;
+  lift_s[t] = 0.0;
+  __syncthreads();
+  double v = 0.0;
+  if (own) {
+    const int i = free_idx[f];
+    const int k0 = row_ptr[i], k1 = row_ptr[i + 1];
+    const bool need = !(rhs_fixed && rhs_fixed[i]);
     if (src) v += 1.0 * src[i];
     if (rhs) v += rhs[i];
-    need = !(rhs_fixed && rhs_fixed[i]);
-  }
-  unsigned long long mask = __ballot(need);
-  while (mask) {
-    const int l = __ffsll((long long)mask) - 1;
-    mask &= mask - 1;
-    const int il = __shfl(i, l, 64);
-    double lift = 0.0;
-    for (int k = row_ptr[il] + lane; k < row_ptr[il + 1]; k += 64) {
-      const int j = col[k];
-      if (new_idx[j] < 0) {
-        const double uj = u[j], kv = vals[k];
-        if (fabs(uj) >= ZT && fabs(kv) >= ZT) lift += -1.0 * kv * uj;
-      }
+    if (need) {  // any order: the rows' sums are independent
+      const int p = atomicAdd(&count, 1);
+      k0s[p] = k0;
+      k1s[p] = k1;
+      who[p] = t;
     }
-    lift = wave_sum(lift);
-    if (lane == l) mine = lift;
   }
-  if (f < n_free) b[f] = v + mine;
+  __syncthreads();
+  const int listed = count;
+  for (int l = t >> 4; l < listed; l += 16) {
+    const int e = k1s[l];
+    double lift = 0.0;
+    for (int k = k0s[l] + sub; k < e; k += 64) {
+      // every entry's value, DOF number and u, used or not: no load waits for another
+      // one's test
+      int j[4], fix[4];
+      double kv[4], uj[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int kq = min(k + 16 * q, e - 1);
+        j[q] = col[kq];
+        kv[q] = vals[kq];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        fix[q] = new_idx[j[q]];
+        uj[q] = u[j[q]];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (k + 16 * q < e && fix[q] < 0 && fabs(uj[q]) >= ZT && fabs(kv[q]) >= ZT) lift += -1.0 * kv[q] * uj[q];
+    }
+    lift = sum16(lift);
+    if (sub == 0) lift_s[who[l]] = lift;
+  }
+  __syncthreads();
+  if (own) b[f] = v + lift_s[t];
 }
 
 __global__ void field_update_kernel(int n_free, const int32_t* __restrict__ free_idx, const double* __restrict__ x,
@@ -121,10 +154,16 @@ __global__ void field_update_kernel(int n_free, const int32_t* __restrict__ free
 }
 
 // R_i = sum_k K_ik u_j - s_i for the rows whose RHS DOF is free (R_i = -s_i for
-// the others).  kBacksubLanes lanes share a row, each summing a strided part of
-// it four entries per trip (the SpMV's row_partial); the parts meet by shuffles
-// inside the lane group.  Rows are dealt over a resident grid.
-constexpr int kBacksubLanes = 16;
+// the others).  Bound by HBM: 12 B per entry.  A block takes kBsRows rows, whose
+// entries are one contiguous range, and reads them tile by tile with all its lanes,
+// eight entries in flight per thread, into LDS (as products K_ik u_j); eight lanes
+// per row then add the row's part of the tile.  Reading row by row with 16 lanes
+// split every load into four misaligned pieces: 75 x 83 x 67 nodes (25.9 M entries, 311
+// and 207 MB for K u and the in-row form), average of both 84 us, now 66 us; 97^3
+// nodes (57 M entries) K u 257 us, now 170 us.  Tiles of 1,024 entries, or loads one
+// tile ahead, measured 9 to 15% slower.
+constexpr int kBsRows = 32;
+constexpr int kBsTile = 2048;
 
 __global__ __launch_bounds__(256) void backsub_kernel(int n, const int32_t* __restrict__ row_ptr,
                                                       const int32_t* __restrict__ col,
@@ -132,25 +171,48 @@ __global__ __launch_bounds__(256) void backsub_kernel(int n, const int32_t* __re
                                                       const double* __restrict__ src,
                                                       const uint8_t* __restrict__ rhs_fixed, int iron_compat,
                                                       double* __restrict__ R) {
-  constexpr int L = kBacksubLanes;
-  const int gpb = blockDim.x / L, sub = threadIdx.x % L;
-  for (int i = blockIdx.x * gpb + threadIdx.x / L; i < n; i += gridDim.x * gpb) {
-    // the row bounds, the fixed flag and the source are independent loads; a
-    // fixed row becomes an empty one
-    const int k0 = row_ptr[i];
-    int k1 = row_ptr[i + 1];
-    if (rhs_fixed && rhs_fixed[i]) k1 = k0;
-    double acc = 0.0;
+  __shared__ double prod[kBsTile];
+  constexpr int U = kBsTile / 256;
+  const int r0 = blockIdx.x * kBsRows, row = r0 + (threadIdx.x >> 3), sub = threadIdx.x & 7;
+  const int e0 = row_ptr[r0], e1 = row_ptr[min(r0 + kBsRows, n)];
+  int a = 0, e = 0;
+  double s = 0.0, acc = 0.0;
+  if (row < n) {
+    a = row_ptr[row];
+    e = row_ptr[row + 1];
+    if (rhs_fixed && rhs_fixed[row]) e = a;  // an empty row
+    if (src) s = src[row];
+  }
+  for (int t0 = e0; t0 < e1; t0 += kBsTile) {
+    const int k = t0 + threadIdx.x, left = e1 - k;
+    double kv[U];
+    if (iron_compat) {
+#pragma unroll
+      for (int q = 0; q < U; ++q) kv[q] = 256 * q < left ? stream_load(&vals[k + 256 * q]) : 0.0;
+    } else {
+      int c[U];
+#pragma unroll
+      for (int q = 0; q < U; ++q) c[q] = 256 * q < left ? stream_load(&col[k + 256 * q]) : 0;
+#pragma unroll
+      for (int q = 0; q < U; ++q) kv[q] = 256 * q < left ? stream_load(&vals[k + 256 * q]) : 0.0;
+#pragma unroll
+      for (int q = 0; q < U; ++q) kv[q] *= u[c[q]];
+    }
+#pragma unroll
+    for (int q = 0; q < U; ++q) prod[threadIdx.x + 256 * q] = kv[q];
+    __syncthreads();
+    const int hi = min(e, t0 + kBsTile);
     if (iron_compat) {
       // equations_set_routines.F90:1806 reads the dependent value at the position
       // within the row; the correct product reads it at the column.
-      for (int k = k0 + sub; k < k1; k += L) acc += vals[k] * u[k - k0];
+      for (int j = max(a, t0) + sub; j < hi; j += 8) acc += prod[j - t0] * u[j - a];
     } else {
-      acc = row_range_partial<double, L>(k0, k1, col, vals, u, sub);
+      for (int j = max(a, t0) + sub; j < hi; j += 8) acc += prod[j - t0];
     }
-    acc = group_sum<double, L>(acc);
-    if (sub == 0) R[i] = acc - (src ? src[i] : 0.0);
+    if (t0 + kBsTile < e1) __syncthreads();
   }
+  acc = sum8(acc);
+  if (row < n && sub == 0) R[row] = acc - s;
 }
 
 // One wavefront per slice: base = min column of the slice, 16-bit offsets, and
@@ -371,7 +433,7 @@ int mife_solver_rhs(int n_free, const int32_t* free_idx, const int32_t* row_ptr,
   MIFE_REQUIRE(free_idx && row_ptr && col && vals && new_idx && u && b, MIFE_ERR_POINTER_IS_NULL,
                "null pointer argument");
   hipStream_t s = (hipStream_t)stream;
-  solver_rhs_kernel<<<div_up(n_free, 256), 256, 0, s>>>(n_free, free_idx, row_ptr, col, vals, new_idx, u, src, rhs,
+  solver_rhs_kernel<<<div_up(n_free, kRhsRows), 256, 0, s>>>(n_free, free_idx, row_ptr, col, vals, new_idx, u, src, rhs,
                                                         rhs_fixed, b);
   MIFE_CHECK_HIP(hipGetLastError());
   return MIFE_OK;
@@ -389,8 +451,7 @@ int mife_backsubstitute(int n, const int32_t* row_ptr, const int32_t* col, const
                         const double* src, const uint8_t* rhs_fixed, int iron_compat, double* R, void* stream) {
   if (n == 0) return MIFE_OK;  // empty arrays may be passed as NULL
   MIFE_REQUIRE(row_ptr && col && vals && u && R, MIFE_ERR_POINTER_IS_NULL, "null pointer argument");
-  const int grid = std::max(1, std::min(div_up(n, 256 / kBacksubLanes), kMaxGrid));
-  backsub_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(n, row_ptr, col, vals, u, src, rhs_fixed, iron_compat, R);
+  backsub_kernel<<<div_up(n, kBsRows), 256, 0, (hipStream_t)stream>>>(n, row_ptr, col, vals, u, src, rhs_fixed, iron_compat, R);
   MIFE_CHECK_HIP(hipGetLastError());
   return MIFE_OK;
 }
