@@ -52,6 +52,26 @@ __device__ __forceinline__ void add_value(T* p, T v, bool atomic) {
   else *p += v;
 }
 
+// N entries of one element into the CSR values (p < 0: none).  They are distinct
+// entries and no other element of the launch touches them (atomic: they may), so every
+// value is loaded before the first is stored: one round trip instead of N (a 23 x 19 x 21
+// triquadratic mesh, eight colour launches: 219 -> 180 us).
+template <typename T, int N>
+__device__ __forceinline__ void add_values(T* __restrict__ vals, const int (&p)[N], const T (&v)[N], bool atomic) {
+  if (atomic) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if (p[k] >= 0) atomicAdd(&vals[p[k]], v[k]);
+    return;
+  }
+  T old[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) old[k] = p[k] >= 0 ? vals[p[k]] : (T)0;
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    if (p[k] >= 0) vals[p[k]] = old[k] + v[k];
+}
+
 // Stage layout of a structured (grid) assembly.  With row m = (c, a), column
 // n = (c2, b), node a = (ax, ay, az) on the element's NB^3 lattice and element
 // e = ex + nx (ey + ny ez), entry (m, n) of element e sits at
@@ -84,11 +104,12 @@ struct GridStripe {
     if (nx <= 0) return blockIdx.x;
     return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   }
-  // block-wide store of the LDS slots K (sbase[w] < 0: wavefront w holds no element)
+  // block-wide store of the LDS slots K of WPB elements (sbase[w] < 0: element slot w
+  // is empty)
   template <typename T, int WPB>
   static __device__ __forceinline__ void store(const T* K, const long long* sbase, int nx, T* stage) {
     const long long stride = (long long)nx * B2;
-    for (int f = threadIdx.x; f < SU * WPB * B2; f += 64 * WPB) {
+    for (int f = threadIdx.x; f < SU * WPB * B2; f += blockDim.x) {
       const int u = f / (WPB * B2), r = f - u * (WPB * B2), w = r / B2, j = r - w * B2;
       const long long b = sbase[w];
       if (b >= 0) stage[b + u * stride + j] = K[f];
@@ -159,7 +180,7 @@ struct ScalarJob {
   const int32_t* edofs;
   const double* kappa;
   const double* source;
-  const int32_t* pos;   // NULL: stage the element matrix at vals[e][NN][NN]
+  const int32_t* pos;   // NULL: structured (the element matrices go to the stage at vals)
   T* vals;
   double* svec;
   double* sstage;       // non-NULL: stage the element source vector at sstage[e][NN]
@@ -167,18 +188,12 @@ struct ScalarJob {
 };
 
 // One element per wavefront (element e when `active`); every wavefront of the
-// block calls it the same number of times (it holds block barriers).  GRID: the
-// element matrix is stored (not added) in the grid stage (GridStripe) for the
-// row-gather pass of a structured assembly.
-template <int DIM, int NN, int NG, typename T, int WPB, bool GRID = false>
+// block calls it the same number of times (it holds block barriers).
+template <int DIM, int NN, int NG, typename T, int WPB>
 __device__ __forceinline__ void scalar_element(const ScalarJob<T>& J, long long e, bool active,
                                                const double* __restrict__ dN, const double* __restrict__ N,
                                                const double* __restrict__ w, bool atomic) {
   constexpr int KD = NG * DIM;
-  static_assert(!GRID || DIM == 3, "the grid assembly is 3-D");
-  using GS = GridStripe<(DIM == 3 ? NN : 8), 1>;
-  __shared__ T sK[GRID ? WPB * NN * NN : 1];
-  __shared__ long long sbase[WPB];
   __shared__ GeomLDS<DIM, NN, NG> geo[WPB];
   __shared__ T sB[WPB][KD * NN];
   __shared__ T sW[WPB][KD];
@@ -208,46 +223,156 @@ __device__ __forceinline__ void scalar_element(const ScalarJob<T>& J, long long 
       T acc = 0;
 #pragma unroll 9
       for (int k = 0; k < KD; ++k) acc += W[k] * B[k * NN + m] * B[k * NN + n];
-      if constexpr (GRID)
-        sK[GS::slot(m, n, wv, WPB)] = acc;
-      else
-        add_value(&J.vals[J.pos[e * (NN * NN) + t]], acc, atomic);
+      add_value(&J.vals[J.pos[e * (NN * NN) + t]], acc, atomic);
     }
-    if (J.source && (J.svec || J.sstage) && lane < NN) {
+    if (J.source && J.svec && lane < NN) {
       // Rounded product and sum, unfused whatever the caller inlines around them
       // (a kernel whose `atomic` is a constant would otherwise fuse them).
 #pragma clang fp contract(off)
       double s = 0.0;
       for (int g = 0; g < NG; ++g) s = fma(N[g * NN + lane], G.rwg[g], s);
       s = s * J.source[e];
-      if (J.sstage)
-        J.sstage[e * NN + lane] = s;
-      else
-        add_value(&J.svec[J.edofs[e * NN + lane]], s, atomic);
+      add_value(&J.svec[J.edofs[e * NN + lane]], s, atomic);
     }
-  }
-  if constexpr (GRID) {
-    if (lane == 0) sbase[wv] = active ? GS::base(e, J.gnx, J.gny) : -1;
-    __syncthreads();
-    GS::template store<T, WPB>(sK, sbase, J.gnx, J.vals);
   }
 }
 
-template <int DIM, int NN, int NG, typename T, int WPB, bool GRID = false>
+template <int DIM, int NN, int NG, typename T, int WPB>
 __global__ __launch_bounds__(64 * WPB) void scalar_assemble_kernel(
     const double* __restrict__ coords, const int32_t* __restrict__ enodes, const int32_t* __restrict__ edofs,
     const double* __restrict__ kappa, const double* __restrict__ source, const int32_t* __restrict__ pos,
     const int32_t* __restrict__ order, int elem_begin, int elem_count, const double* __restrict__ dN,
     const double* __restrict__ N, const double* __restrict__ w, T* __restrict__ vals, double* __restrict__ svec,
-    bool atomic, double* __restrict__ sstage = nullptr, int gnx = 0, int gny = 0) {
-  const int blk = GRID ? GridStripe<NN, 1>::block(gnx) : (int)blockIdx.x;
-  const int idx = blk * WPB + (threadIdx.x >> 6);
+    bool atomic) {
+  const int idx = (int)blockIdx.x * WPB + (threadIdx.x >> 6);
   const bool active = idx < elem_count;
   long long e = 0;
   if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
-  scalar_element<DIM, NN, NG, T, WPB, GRID>(
-      ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec, sstage, gnx, gny}, e, active, dN, N, w,
+  scalar_element<DIM, NN, NG, T, WPB>(
+      ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec, nullptr, 0, 0}, e, active, dN, N, w,
       atomic);
+}
+
+// ------------------------------------------------ trilinear elements, eight per wavefront
+// A wavefront integrates eight elements: lane = (element, Gauss point) forms dx/dxi,
+// its inverse and the point's physical gradients in registers, and the eight points'
+// contributions to an entry meet by DPP inside the element's eight lanes.  With one
+// element per wavefront only 16 of 64 lanes formed geometry, and the sums read 72 LDS
+// values per entry.  All forms (structured, coloured, batched) run this code, with
+// every multiply-add written out, so their sums agree bit for bit.
+constexpr int kQ1Elems = 32;  // elements per block of 256 threads
+
+struct Q1Tables {
+  double dN[8 * 8 * 3];
+  double X[kQ1Elems][8][3];
+};
+
+// Geometry of lane's (element, Gauss point q): ji[j][i] = dxi_j/dx_i, and |J| w_q.
+// Holds two block barriers.
+__device__ __forceinline__ double q1_geometry(Q1Tables& S, const double* __restrict__ coords,
+                                              const int32_t* __restrict__ enodes, long long e, bool active,
+                                              const double* __restrict__ dN, const double* __restrict__ w,
+                                              double (&ji)[3][3]) {
+  const int el = threadIdx.x >> 3, q = threadIdx.x & 7;
+  __syncthreads();  // the tables of an earlier pass are done with
+  if (threadIdx.x < 8 * 8 * 3) S.dN[threadIdx.x] = dN[threadIdx.x];
+  if (active) {
+    const long long node = enodes[e * 8 + q];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) S.X[el][q][d] = coords[node * 3 + d];
+  }
+  __syncthreads();
+  double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+  for (int a = 0; a < 8; ++a)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const double dn = S.dN[(q * 8 + a) * 3 + j];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) J[d][j] = fma(S.X[el][a][d], dn, J[d][j]);
+    }
+  const double det = invert<3>(J, ji);
+  return fabs(det) * w[q];
+}
+
+// One scalar element per eight lanes (e and J are the eight lanes' own); every thread
+// of the block calls it.
+template <typename T, bool GRID>
+__device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, long long e, bool active,
+                                                   const double* __restrict__ dN, const double* __restrict__ N,
+                                                   const double* __restrict__ w, bool atomic) {
+#pragma clang fp contract(off)
+  using GS = GridStripe<8, 1>;
+  __shared__ Q1Tables S;
+  __shared__ double rw[kQ1Elems][8];
+  __shared__ T sK[kQ1Elems * 64];
+  __shared__ long long sbase[kQ1Elems];
+  const int el = threadIdx.x >> 3, q = threadIdx.x & 7;
+  double ji[3][3];
+  const double rwg = q1_geometry(S, J.coords, J.enodes, e, active, dN, w, ji);
+  const double ke = (active && J.kappa) ? J.kappa[e] : 1.0;
+  const T W = (T)(rwg * ke);
+  T B[8][3];
+#pragma unroll
+  for (int a = 0; a < 8; ++a) {
+    const double* d = &S.dN[(q * 8 + a) * 3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) B[a][i] = (T)fma(d[0], ji[0][i], fma(d[1], ji[1][i], d[2] * ji[2][i]));
+  }
+  rw[el][q] = rwg;
+  int t = 0;
+#pragma unroll
+  for (int m = 0; m < 8; ++m) {
+    const T b0 = W * B[m][0], b1 = W * B[m][1], b2 = W * B[m][2];
+#pragma unroll
+    for (int n = m; n < 8; ++n, ++t) {
+      const T v = sum8(fma(b0, B[n][0], fma(b1, B[n][1], b2 * B[n][2])));
+      if (q == (t & 7)) {  // entry t of the upper triangle, and its transpose
+        sK[GRID ? GS::slot(m, n, el, kQ1Elems) : el * 64 + m * 8 + n] = v;
+        sK[GRID ? GS::slot(n, m, el, kQ1Elems) : el * 64 + n * 8 + m] = v;
+      }
+    }
+  }
+  if (GRID && q == 0) sbase[el] = active ? GS::base(e, J.gnx, J.gny) : -1;
+  __syncthreads();
+  if constexpr (GRID) {
+    GS::template store<T, kQ1Elems>(sK, sbase, J.gnx, J.vals);
+  } else if (active) {
+    const int32_t* pe = J.pos + e * 64 + q * 8;
+    int p[8];
+    T v[8];
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      p[n] = pe[n];
+      v[n] = sK[el * 64 + q * 8 + n];
+    }
+    add_values(J.vals, p, v, atomic);
+  }
+  if (active && J.source && (J.svec || J.sstage)) {
+    double s = 0.0;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) s = fma(N[g * 8 + q], rw[el][g], s);
+    s = s * J.source[e];
+    if (J.sstage)
+      J.sstage[e * 8 + q] = s;
+    else
+      add_value(&J.svec[J.edofs[e * 8 + q]], s, atomic);
+  }
+}
+
+// Measured on 61 x 47 x 53 elements with moved nodes, FP64, structured: 187 us with
+// one element per wavefront, 55 us now (78 MB of element matrices stored).
+template <typename T, bool GRID>
+__global__ __launch_bounds__(256) void q1_scalar_kernel(ScalarJob<T> J, const int32_t* __restrict__ order,
+                                                        int elem_begin, int elem_count,
+                                                        const double* __restrict__ dN, const double* __restrict__ N,
+                                                        const double* __restrict__ w, bool atomic) {
+  const int blk = GRID ? GridStripe<8, 1>::block(J.gnx) : (int)blockIdx.x;
+  const int idx = blk * kQ1Elems + (threadIdx.x >> 3);
+  const bool active = idx < elem_count;
+  long long e = 0;
+  if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
+  q1_scalar_elements<T, GRID>(J, e, active, dN, N, w, atomic);
 }
 
 // ------------------------------------------------ triquadratic, on MFMA
@@ -278,14 +403,19 @@ struct Mfma16<float> {
   static __device__ __forceinline__ int row(int lane, int i) { return 4 * (lane >> 4) + i; }
 };
 
-template <typename T, int WPB>
-__global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(4))) void q2_assemble_mfma_kernel(
+// GRID: the element matrices go to the stage (four wavefronts per SIMD hide the
+// operand formation); else they are added into the CSR values, 16 entries per lane at
+// once, which takes the registers of two.
+constexpr int kQ2Waves = 4;
+
+template <typename T, bool GRID>
+__global__ __launch_bounds__(64 * kQ2Waves) __attribute__((amdgpu_waves_per_eu(GRID ? 4 : 2))) void q2_assemble_mfma_kernel(
     const double* __restrict__ coords, const int32_t* __restrict__ enodes, const int32_t* __restrict__ edofs,
     const double* __restrict__ kappa, const double* __restrict__ source, const int32_t* __restrict__ pos,
     const int32_t* __restrict__ order, int elem_begin, int elem_count, const double* __restrict__ dN,
     const double* __restrict__ N, const double* __restrict__ w, T* __restrict__ vals, double* __restrict__ svec,
-    bool atomic, double* __restrict__ sstage = nullptr, int gnx = 0, int gny = 0) {
-  constexpr int NN = 27, NG = 27, KD = 81, STEPS = 21;
+    bool atomic, double* __restrict__ sstage, int gnx, int gny) {
+  constexpr int NN = 27, NG = 27, KD = 81, STEPS = 21, WPB = kQ2Waves;
   using M = Mfma16<T>;
   using GS = GridStripe<NN, 1>;
   // the element matrices of a grid stage reuse the LDS of the reference
@@ -310,7 +440,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(4))) v
   if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
   GeomLDS<3, NN, NG>& G = sh.t.geo[wv];
   element_geometry<3, NN, NG>(G, coords, enodes, e, sdN, w, lane, active);
-  if (pos && !active) return;  // the scatter holds no further barrier
+  if (!GRID && !active) return;  // the scatter holds no further barrier
   const int kq = lane >> 4, col = lane & 15;
   typename M::v4 k00 = {0, 0, 0, 0}, k01 = {0, 0, 0, 0}, k11 = {0, 0, 0, 0};
   double s = 0.0;
@@ -337,21 +467,25 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(4))) v
       s *= source[e];
     }
   }
-  if (pos) {
+  if constexpr (!GRID) {
     const int32_t* pe = pos + e * (NN * NN);
+    const bool second = 16 + col < NN;
+    int p[16];
+    T v[16];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = M::row(lane, i);
-      // tile (0,0): m = r, n = col
-      add_value(&vals[pe[r * NN + col]], k00[i], atomic);
-      // tile (0,1) and its transpose: m = r, n = 16 + col
-      if (16 + col < NN) {
-        add_value(&vals[pe[r * NN + 16 + col]], k01[i], atomic);
-        add_value(&vals[pe[(16 + col) * NN + r]], k01[i], atomic);
-      }
+      // tile (0,0): m = r, n = col; tile (0,1) and its transpose: n = 16 + col;
       // tile (1,1): m = 16 + r, n = 16 + col
-      if (16 + r < NN && 16 + col < NN) add_value(&vals[pe[(16 + r) * NN + 16 + col]], k11[i], atomic);
+      p[4 * i] = pe[r * NN + col];
+      p[4 * i + 1] = second ? pe[r * NN + 16 + col] : -1;
+      p[4 * i + 2] = second ? pe[(16 + col) * NN + r] : -1;
+      p[4 * i + 3] = second && 16 + r < NN ? pe[(16 + r) * NN + 16 + col] : -1;
+      v[4 * i] = k00[i];
+      v[4 * i + 1] = v[4 * i + 2] = k01[i];
+      v[4 * i + 3] = k11[i];
     }
+    add_values(vals, p, v, atomic);
     if (source && svec && lane < NN) add_value(&svec[edofs[e * NN + lane]], s, atomic);
     return;
   }
@@ -377,94 +511,15 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(4))) v
 }
 
 // ------------------------------------------------------- linear elasticity
-// Iron's per-block coefficient use (linear_elasticity_routines.F90:1255-1286):
-// diagonal block c uses JRWG*diagC[c][d] on dphi_d*dphi_d; off-diagonal block
-// (c1<c2) uses Ca*dphi_n,c1*dphi_m,c2 + Cb*dphi_n,c2*dphi_m,c1.
-template <int NN, int NG, typename T, int WPB>
-__global__ __launch_bounds__(64 * WPB) void elastic_assemble_kernel(
-    const double* __restrict__ coords, const int32_t* __restrict__ enodes, const double* __restrict__ material,
-    const int32_t* __restrict__ pos, const int32_t* __restrict__ order, int elem_begin, int elem_count,
-    const double* __restrict__ dN, const double* __restrict__ w, T* __restrict__ vals, bool atomic) {
-  constexpr int ND = 3 * NN;
-  __shared__ GeomLDS<3, NN, NG> geo[WPB];
-  __shared__ T sB[WPB][NG][NN][3];
-  __shared__ T sC[WPB][NG][12];  // per GP: diag[3][3] (9) + off Ca,Cb handled below
-  __shared__ T sOff[WPB][NG][6];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int idx = blockIdx.x * WPB + wv;
-  const bool active = idx < elem_count;
-  long long e = 0;
-  if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
-  GeomLDS<3, NN, NG>& G = geo[wv];
-  element_geometry<3, NN, NG>(G, coords, enodes, e, dN, w, lane, active);
-  if (active) {
-    for (int t = lane; t < NG * NN; t += 64) {
-      const int g = t / NN, a = t - (t / NN) * NN;
-      // dphidx(a,mi) = sum_ni DXI_DX(mi,ni) dphi/dxi_ni   (linear_elasticity_routines.F90:1245-1252)
-#pragma unroll
-      for (int mi = 0; mi < 3; ++mi) {
-        double b = 0.0;
-#pragma unroll
-        for (int ni = 0; ni < 3; ++ni) b += G.ji[g][mi][ni] * dN[(g * NN + a) * 3 + ni];
-        sB[wv][g][a][mi] = (T)b;
-      }
-    }
-    if (lane < NG) {
-      const int g = lane;
-      const double* mat = material + e * 6;
-      const double E1 = mat[0], E2 = mat[1], E3 = mat[2], v13 = mat[3], v23 = mat[4], v12 = mat[5];
-      const double v31 = v13, v32 = v23, v21 = v12;
-      const double gama = 1.0 / (1.0 - v12 * v21 - v23 * v32 - v31 * v13 - 2.0 * v21 * v32 * v13);
-      const double C11 = E1 * (1.0 - v23 * v32) * gama, C22 = E2 * (1.0 - v13 * v31) * gama;
-      const double C33 = E3 * (1.0 - v12 * v21) * gama;
-      const double C12 = E1 * (v21 + v31 * v23) * gama, C13 = E1 * (v31 + v21 * v32) * gama;
-      const double C23 = E2 * (v32 + v12 * v31) * gama;
-      const double C44 = E2 / (2.0 * (1.0 + v23)), C55 = E1 / (2.0 * (1.0 + v13)), C66 = E3 / (2.0 * (1.0 + v12));
-      const double jr = G.rwg[g];
-      const double diag[9] = {C11, C66, C44, C66, C22, C55, C44, C55, C33};
-      for (int k = 0; k < 9; ++k) sC[wv][g][k] = (T)(jr * diag[k]);
-      const double off[6] = {C12, C66, C13, C44, C23, C55};
-      for (int k = 0; k < 6; ++k) sOff[wv][g][k] = (T)(jr * off[k]);
-    }
-  }
-  __syncthreads();
-  if (active) {
-    for (int t = lane; t < ND * ND; t += 64) {
-      const int r = t / ND, s = t - (t / ND) * ND;
-      int c1 = r / NN, n = r - (r / NN) * NN;
-      int c2 = s / NN, m = s - (s / NN) * NN;
-      T acc = 0;
-      if (c1 == c2) {
-        for (int g = 0; g < NG; ++g) {
-          const T* D = &sC[wv][g][c1 * 3];
-          acc += D[0] * sB[wv][g][n][0] * sB[wv][g][m][0] + D[1] * sB[wv][g][n][1] * sB[wv][g][m][1] +
-                 D[2] * sB[wv][g][n][2] * sB[wv][g][m][2];
-        }
-      } else {
-        // order the pair so that (c1 < c2); the lower blocks are the transpose
-        if (c1 > c2) {
-          int tc = c1; c1 = c2; c2 = tc;
-          int tn = n; n = m; m = tn;
-        }
-        const int blk = (c1 == 0) ? (c2 == 1 ? 0 : 1) : 2;
-        for (int g = 0; g < NG; ++g) {
-          const T Ca = sOff[wv][g][2 * blk], Cb = sOff[wv][g][2 * blk + 1];
-          acc += Ca * sB[wv][g][n][c1] * sB[wv][g][m][c2] + Cb * sB[wv][g][n][c2] * sB[wv][g][m][c1];
-        }
-      }
-      const int p = pos[e * (ND * ND) + t];
-      add_value(&vals[p], acc, atomic);
-    }
-  }
-}
-
-// Trilinear elasticity on MFMA: K[(i,a)][(j,b)] = sum_g sum_L U[(i,j,a)][(g,L)]
-// B[g][b][L], one (9 NN) x (3 NG) by (3 NG) x NN GEMM per element (one
-// wavefront per element, 16x16x4 tiles).  U carries iron's per-block
-// coefficients: U[(c,c,a)][(g,L)] = w diagC[c][L] B[g][a][L] on the diagonal
-// blocks and, for i != j, U[(i,j,a)][(g,L)] = w (Ca B[g][a][i] [L == j] +
-// Cb B[g][a][j] [L == i]) with (Ca, Cb) of the pair {i, j}
-// (linear_elasticity_routines.F90:1255-1286; the lower blocks are the transposes).
+// Trilinear elasticity.  The coefficients are constant over an element, so its 24 x 24
+// matrix is a combination of the nine products S_kl[n][m] = sum_g w_g B[g][n][k]
+// B[g][m][l]: diagonal block (c,c) is sum_k diagC[c][k] S_kk, and block (i,j) with
+// the pair's (Ca, Cb) is Ca S_ij + Cb S_ji for i < j (linear_elasticity_routines.F90:
+// 1255-1286; the lower blocks are the transposes).  A wavefront forms the gradients of
+// eight elements, lane = (element, Gauss point), and then takes the elements in turn,
+// lane = node pair (n, m): nine sums in registers, 72 multiply-adds, from which the
+// lane's nine entries follow.  As one GEMM on MFMA with the coefficients inside the
+// operands the same matrix took 30 tile steps and as many LDS-formed operands.
 template <typename T>
 struct ElasticJob {
   const double* coords;
@@ -475,117 +530,137 @@ struct ElasticJob {
   int gnx, gny;  // GRID: elements in x and y (GridStripe layout)
 };
 
-// GRID: every wavefront of the block must call it (it ends with block barriers);
-// the element matrix goes to the grid stage (GridStripe) instead of the CSR.
-template <typename T, int NN, int NG, int WPB, bool GRID = false>
-__device__ __forceinline__ void elastic_element(const ElasticJob<T>& J, long long e, bool active,
-                                                const double* __restrict__ dN, const double* __restrict__ w,
-                                                bool atomic) {
-  constexpr int ND = 3 * NN, MROWS = 9 * NN, KD = 3 * NG;
-  constexpr int MT = (MROWS + 15) / 16, STEPS = (KD + 3) / 4;
-  static_assert(NN <= 16, "one column tile");
-  using M = Mfma16<T>;
-  using GS = GridStripe<NN, 3>;
-  __shared__ T sK[GRID ? WPB * ND * ND : 1];
-  __shared__ long long sbase[WPB];
-  __shared__ GeomLDS<3, NN, NG> geo[WPB];
-  __shared__ T sB[WPB][NG][NN][3];
-  __shared__ T sDiag[WPB][NG][9];  // w * diagC[c][d]
-  __shared__ T sOff[WPB][NG][6];   // w * (Ca, Cb) of the pairs (0,1), (0,2), (1,2)
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  GeomLDS<3, NN, NG>& G = geo[wv];
-  element_geometry<3, NN, NG>(G, J.coords, J.enodes, e, dN, w, lane, active);
-  if (active) {
-    for (int t = lane; t < NG * NN; t += 64) {
-      const int g = t / NN, a = t - (t / NN) * NN;
-      // dphidx(a,mi) = sum_ni DXI_DX(mi,ni) dphi/dxi_ni   (linear_elasticity_routines.F90:1245-1252)
+// Element 4 i + w of a block belongs to wavefront w (lanes 8 i .. 8 i + 7 hold its
+// number and arrays): in turn i the four wavefronts take consecutive elements, whose
+// entries leave through LDS in runs of 16 values.  Half of the gradients are in LDS
+// at a time, which keeps two blocks on a CU.
+__device__ __forceinline__ int q1_elastic_slot() { return 4 * ((threadIdx.x & 63) >> 3) + (threadIdx.x >> 6); }
+
+template <typename T, bool GRID>
+__device__ __forceinline__ void q1_elastic_elements(const ElasticJob<T>& J, long long e, bool active,
+                                                    const double* __restrict__ dN, const double* __restrict__ w,
+                                                    bool atomic) {
+#pragma clang fp contract(off)
+  using GS = GridStripe<8, 3>;
+  constexpr int kWaves = kQ1Elems / 8, kHalf = 4, kRun = kWaves * GS::B2;
+  __shared__ Q1Tables S;
+  __shared__ T sB[kWaves][kHalf][8][8][3];
+  __shared__ T sW[kWaves][8][8];
+  __shared__ T sC[kWaves][8][15];  // diagC[3][3], then (Ca, Cb) of the pairs (0,1), (0,2), (1,2)
+  __shared__ T sK[GRID ? 2 : 1][GRID ? GS::SU * kRun : 1];
+  __shared__ long long sbase[kWaves][8];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i8 = lane >> 3, q = lane & 7;
+  double ji[3][3];
+  const double rwg = q1_geometry(S, J.coords, J.enodes, e, active, dN, w, ji);
+  T B[8][3];
 #pragma unroll
-      for (int mi = 0; mi < 3; ++mi) {
-        double b = 0.0;
+  for (int a = 0; a < 8; ++a) {
+    const double* d = &S.dN[(q * 8 + a) * 3];
+    // dphidx(a,mi) = sum_ni DXI_DX(mi,ni) dphi/dxi_ni   (linear_elasticity_routines.F90:1245-1252)
 #pragma unroll
-        for (int ni = 0; ni < 3; ++ni) b += G.ji[g][mi][ni] * dN[(g * NN + a) * 3 + ni];
-        sB[wv][g][a][mi] = (T)b;
-      }
-    }
-    if (lane < NG) {
-      const int g = lane;
-      const double* mat = J.material + e * 6;
-      const double E1 = mat[0], E2 = mat[1], E3 = mat[2], v13 = mat[3], v23 = mat[4], v12 = mat[5];
-      const double v31 = v13, v32 = v23, v21 = v12;
-      const double gama = 1.0 / (1.0 - v12 * v21 - v23 * v32 - v31 * v13 - 2.0 * v21 * v32 * v13);
-      const double C11 = E1 * (1.0 - v23 * v32) * gama, C22 = E2 * (1.0 - v13 * v31) * gama;
-      const double C33 = E3 * (1.0 - v12 * v21) * gama;
-      const double C12 = E1 * (v21 + v31 * v23) * gama, C13 = E1 * (v31 + v21 * v32) * gama;
-      const double C23 = E2 * (v32 + v12 * v31) * gama;
-      const double C44 = E2 / (2.0 * (1.0 + v23)), C55 = E1 / (2.0 * (1.0 + v13)), C66 = E3 / (2.0 * (1.0 + v12));
-      const double jr = G.rwg[g];
-      const double diag[9] = {C11, C66, C44, C66, C22, C55, C44, C55, C33};
-      for (int k = 0; k < 9; ++k) sDiag[wv][g][k] = (T)(jr * diag[k]);
-      const double off[6] = {C12, C66, C13, C44, C23, C55};
-      for (int k = 0; k < 6; ++k) sOff[wv][g][k] = (T)(jr * off[k]);
-    }
+    for (int mi = 0; mi < 3; ++mi) B[a][mi] = (T)fma(ji[mi][0], d[0], fma(ji[mi][1], d[1], ji[mi][2] * d[2]));
   }
-  __syncthreads();
-  if (!GRID && !active) return;  // the scatter holds no further barrier
-  const int32_t* pe = GRID ? nullptr : J.pos + e * (ND * ND);
-  const int col = lane & 15;
-  for (int mt = 0; active && mt < MT; ++mt) {
-    const int mrow = 16 * mt + col;
-    const bool rv = mrow < MROWS;
-    const int i = rv ? mrow / (3 * NN) : 0, j = rv ? (mrow / NN) % 3 : 0, a = rv ? mrow % NN : 0;
-    const int blk = (i + j == 1) ? 0 : ((i + j == 2) ? 1 : 2);  // pairs (0,1), (0,2), (1,2)
-    typename M::v4 acc = {0, 0, 0, 0};
+  sW[wv][i8][q] = (T)rwg;
+  if (q == 0) sbase[wv][i8] = GRID && active ? GS::base(e, J.gnx, J.gny) : -1;
+  if (q == 0 && active) {
+    const double* mat = J.material + e * 6;
+    const double E1 = mat[0], E2 = mat[1], E3 = mat[2], v13 = mat[3], v23 = mat[4], v12 = mat[5];
+    const double v31 = v13, v32 = v23, v21 = v12;
+    const double gama = 1.0 / (1.0 - v12 * v21 - v23 * v32 - v31 * v13 - 2.0 * v21 * v32 * v13);
+    const double C11 = E1 * (1.0 - v23 * v32) * gama, C22 = E2 * (1.0 - v13 * v31) * gama;
+    const double C33 = E3 * (1.0 - v12 * v21) * gama;
+    const double C12 = E1 * (v21 + v31 * v23) * gama, C13 = E1 * (v31 + v21 * v32) * gama;
+    const double C23 = E2 * (v32 + v12 * v31) * gama;
+    const double C44 = E2 / (2.0 * (1.0 + v23)), C55 = E1 / (2.0 * (1.0 + v13)), C66 = E3 / (2.0 * (1.0 + v12));
+    const double coef[15] = {C11, C66, C44, C66, C22, C55, C44, C55, C33, C12, C66, C13, C44, C23, C55};
 #pragma unroll
-    for (int st = 0; st < STEPS; ++st) {
-      const int k = 4 * st + (lane >> 4);
-      const bool kv = k < KD;
-      const int g = kv ? k / 3 : 0, L = k - 3 * (k / 3);
-      T u = 0, bop = 0;
-      if (kv) {
-        if (rv) {
-          const T* Bg = &sB[wv][g][a][0];
-          if (i == j)
-            u = sDiag[wv][g][i * 3 + L] * Bg[L];
-          else
-            u = (L == j ? sOff[wv][g][2 * blk] * Bg[i] : (T)0) + (L == i ? sOff[wv][g][2 * blk + 1] * Bg[j] : (T)0);
-        }
-        if (col < NN) bop = sB[wv][g][col][L];
-      }
-      acc = M::mac(u, bop, acc);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int orow = 16 * mt + M::row(lane, r);
-      if (orow < MROWS && col < NN) {
-        const int oi = orow / (3 * NN), oj = (orow / NN) % 3, oa = orow % NN;
-        if constexpr (GRID)
-          sK[GS::slot(oi * NN + oa, oj * NN + col, wv, WPB)] = acc[r];
-        else
-          add_value(&J.vals[pe[(oi * NN + oa) * ND + oj * NN + col]], acc[r], atomic);
-      }
-    }
+    for (int k = 0; k < 15; ++k) sC[wv][i8][k] = (T)coef[k];
   }
-  if constexpr (GRID) {
-    if (lane == 0) sbase[wv] = active ? GS::base(e, J.gnx, J.gny) : -1;
+  const int n = lane >> 3, m = lane & 7;
+  const long long stride = (long long)J.gnx * GS::B2;  // GRID
+  for (int half = 0; half < 2; ++half) {
     __syncthreads();
-    GS::template store<T, WPB>(sK, sbase, J.gnx, J.vals);
+    if ((i8 >> 2) == half) {
+#pragma unroll
+      for (int a = 0; a < 8; ++a)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) sB[wv][i8 & 3][q][a][k] = B[a][k];
+    }
+    __syncthreads();
+    for (int h = 0; h < kHalf; ++h) {
+      const int it = kHalf * half + h;
+      const bool on = __builtin_amdgcn_readlane((int)active, 8 * it) != 0;
+      T P[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const T wg = sW[wv][it][g];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const T bn = wg * sB[wv][h][g][n][k];
+#pragma unroll
+          for (int l = 0; l < 3; ++l) P[k][l] = fma(bn, sB[wv][h][g][m][l], P[k][l]);
+        }
+      }
+      const T* C = sC[wv][it];
+      T K[3][3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        K[c][c] = fma(C[3 * c], P[0][0], fma(C[3 * c + 1], P[1][1], C[3 * c + 2] * P[2][2]));
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = i + 1; j < 3; ++j) {
+          const T Ca = C[9 + 2 * (i + j - 1)], Cb = C[10 + 2 * (i + j - 1)];
+          K[i][j] = fma(Ca, P[i][j], Cb * P[j][i]);
+          K[j][i] = fma(Ca, P[j][i], Cb * P[i][j]);
+        }
+      if constexpr (GRID) {
+        T* Ks = sK[it & 1];
+        const int at = ((n >> 1) * 12 + (m >> 1)) * kRun + wv * GS::B2 + (n & 1) * 2 + (m & 1);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int c2 = 0; c2 < 3; ++c2) Ks[at + (48 * c + 4 * c2) * kRun] = K[c][c2];
+        __syncthreads();  // the other buffer is written next: its stores are done by the barrier after
+        const int r = threadIdx.x % kRun, u0 = threadIdx.x / kRun;
+        const long long b = sbase[r / GS::B2][it];
+        if (b >= 0) {
+          T* out = J.vals + b + u0 * stride + r % GS::B2;
+#pragma unroll
+          for (int k = 0; k < GS::SU * kRun / 256; ++k) out[(256 / kRun) * k * stride] = Ks[threadIdx.x + 256 * k];
+        }
+      } else if (on) {
+        const long long ee = lane_value(e, 8 * it);
+        const int32_t* pe = lane_value(J.pos, 8 * it) + ee * 576 + n * 24 + m;
+        T* vals = lane_value(J.vals, 8 * it);
+        int p[9];
+        T v[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+          p[k] = pe[(k / 3) * 192 + (k % 3) * 8];
+          v[k] = K[k / 3][k % 3];
+        }
+        add_values(vals, p, v, atomic);
+      }
+    }
   }
 }
 
 // GRID: a structured assembly's stage (elements in order, gnx x gny per z-layer).
-template <typename T, int NN, int NG, int WPB, bool GRID = false>
-__global__ __launch_bounds__(64 * WPB) void elastic_assemble_mfma_kernel(
-    const double* __restrict__ coords, const int32_t* __restrict__ enodes, const double* __restrict__ material,
-    const int32_t* __restrict__ pos, const int32_t* __restrict__ order, int elem_begin, int elem_count,
-    const double* __restrict__ dN, const double* __restrict__ w, T* __restrict__ vals, bool atomic, int gnx = 0,
-    int gny = 0) {
-  const int blk = GRID ? GridStripe<NN, 3>::block(gnx) : (int)blockIdx.x;
-  const int idx = blk * WPB + (threadIdx.x >> 6);
+// Measured on 63 x 41 x 38 elements with moved nodes, FP64, structured: 337 us as one
+// MFMA GEMM per element, 148 us now (452 MB of element matrices stored); 190 us with the
+// entries stored straight from registers in runs of four values.
+template <typename T, bool GRID>
+__global__ __launch_bounds__(256) void q1_elastic_kernel(ElasticJob<T> J, const int32_t* __restrict__ order,
+                                                         int elem_begin, int elem_count,
+                                                         const double* __restrict__ dN, const double* __restrict__ w,
+                                                         bool atomic) {
+  const int blk = GRID ? GridStripe<8, 3>::block(J.gnx) : (int)blockIdx.x;
+  const int idx = blk * kQ1Elems + q1_elastic_slot();
   const bool active = idx < elem_count;
   long long e = 0;
   if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
-  elastic_element<T, NN, NG, WPB, GRID>(ElasticJob<T>{coords, enodes, material, pos, vals, gnx, gny}, e, active,
-                                        dN, w, atomic);
+  q1_elastic_elements<T, GRID>(J, e, active, dN, w, atomic);
 }
 
 // ------------------------------------------- many meshes in one launch
@@ -593,7 +668,7 @@ __global__ __launch_bounds__(64 * WPB) void elastic_assemble_mfma_kernel(
 // requests a server admits together): one launch per colour and element kind
 // covers every mesh of the batch.  A launch walks a list of segments -- the
 // elements of one colour of one mesh -- as one flattened index space; each
-// wavefront finds its segment by bisection and runs the same element code as
+// element's lanes find its segment by bisection and run the same element code as
 // the one-mesh kernels, so a mesh's values are bit for bit those of its own
 // assembly.  Blocks loop over the index space (a resident grid).
 struct BatchJob {
@@ -629,15 +704,14 @@ __device__ __forceinline__ const BatchSeg& batch_seg(const BatchSeg* __restrict_
   return segs[lo];
 }
 
-template <typename T, int WPB>
-__global__ __launch_bounds__(64 * WPB) void scalar_batch_kernel(const BatchJob* __restrict__ jobs,
-                                                                const BatchSeg* __restrict__ segs, int nseg,
-                                                                int total, const double* __restrict__ dN,
-                                                                const double* __restrict__ N,
-                                                                const double* __restrict__ w) {
-  const int wv = threadIdx.x >> 6;
-  for (int base = blockIdx.x * WPB; base < total; base += gridDim.x * WPB) {
-    const int idx = base + wv;
+template <typename T>
+__global__ __launch_bounds__(256) void scalar_batch_kernel(const BatchJob* __restrict__ jobs,
+                                                           const BatchSeg* __restrict__ segs, int nseg, int total,
+                                                           const double* __restrict__ dN,
+                                                           const double* __restrict__ N,
+                                                           const double* __restrict__ w) {
+  for (int base = blockIdx.x * kQ1Elems; base < total; base += gridDim.x * kQ1Elems) {
+    const int idx = base + (threadIdx.x >> 3);
     const bool active = idx < total;
     ScalarJob<T> J{};
     long long e = 0;
@@ -647,18 +721,17 @@ __global__ __launch_bounds__(64 * WPB) void scalar_batch_kernel(const BatchJob* 
       J = ScalarJob<T>{B.coords, B.enodes, B.edofs, B.coef, B.source, B.pos, (T*)B.vals, B.svec, nullptr, 0, 0};
       e = B.order[sg.begin + idx - sg.prefix];
     }
-    scalar_element<3, 8, 8, T, WPB>(J, e, active, dN, N, w, false);
+    q1_scalar_elements<T, false>(J, e, active, dN, N, w, false);
   }
 }
 
-template <typename T, int WPB>
-__global__ __launch_bounds__(64 * WPB) void elastic_batch_kernel(const BatchJob* __restrict__ jobs,
-                                                                 const BatchSeg* __restrict__ segs, int nseg,
-                                                                 int total, const double* __restrict__ dN,
-                                                                 const double* __restrict__ w) {
-  const int wv = threadIdx.x >> 6;
-  for (int base = blockIdx.x * WPB; base < total; base += gridDim.x * WPB) {
-    const int idx = base + wv;
+template <typename T>
+__global__ __launch_bounds__(256) void elastic_batch_kernel(const BatchJob* __restrict__ jobs,
+                                                            const BatchSeg* __restrict__ segs, int nseg, int total,
+                                                            const double* __restrict__ dN,
+                                                            const double* __restrict__ w) {
+  for (int base = blockIdx.x * kQ1Elems; base < total; base += gridDim.x * kQ1Elems) {
+    const int idx = base + q1_elastic_slot();
     const bool active = idx < total;
     ElasticJob<T> J{};
     long long e = 0;
@@ -668,7 +741,7 @@ __global__ __launch_bounds__(64 * WPB) void elastic_batch_kernel(const BatchJob*
       J = ElasticJob<T>{B.coords, B.enodes, B.coef, B.pos, (T*)B.vals, 0, 0};
       e = B.order[sg.begin + idx - sg.prefix];
     }
-    elastic_element<T, 8, 8, WPB>(J, e, active, dN, w, false);
+    q1_elastic_elements<T, false>(J, e, active, dN, w, false);
   }
 }
 
@@ -679,12 +752,16 @@ static int launch_scalar(const mife_element_desc* d, int n_elem, const double* c
                          hipStream_t s) {
   constexpr int WPB = (sizeof(T) * NG * DIM * NN > 12000) ? 1 : 4;
   constexpr bool kMfma = DIM == 3 && NN == 27 && NG == 27;
-  constexpr int WQ = 4;  // waves (elements) per block of the MFMA kernel
   const int tk = prof::begin(s);
   auto launch = [&](const int32_t* ord, int begin, int count, bool atomic) {
-    if constexpr (kMfma)
-      q2_assemble_mfma_kernel<T, WQ><<<div_up(count, WQ), 64 * WQ, 0, s>>>(
-          coords, enodes, edofs, kappa, source, pos, ord, begin, count, d->dN, d->N, d->w, vals, svec, atomic);
+    if constexpr (DIM == 3 && NN == 8 && NG == 8)
+      q1_scalar_kernel<T, false><<<div_up(count, kQ1Elems), 256, 0, s>>>(
+          ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec, nullptr, 0, 0}, ord, begin, count, d->dN,
+          d->N, d->w, atomic);
+    else if constexpr (kMfma)
+      q2_assemble_mfma_kernel<T, false><<<div_up(count, kQ2Waves), 64 * kQ2Waves, 0, s>>>(
+          coords, enodes, edofs, kappa, source, pos, ord, begin, count, d->dN, d->N, d->w, vals, svec, atomic, nullptr,
+          0, 0);
     else
       scalar_assemble_kernel<DIM, NN, NG, T, WPB><<<div_up(count, WPB), 64 * WPB, 0, s>>>(
           coords, enodes, edofs, kappa, source, pos, ord, begin, count, d->dN, d->N, d->w, vals, svec, atomic);
@@ -702,21 +779,14 @@ static int launch_scalar(const mife_element_desc* d, int n_elem, const double* c
   return MIFE_OK;
 }
 
-template <int NN, int NG, typename T>
+template <typename T>
 static int launch_elastic(const mife_element_desc* d, int n_elem, const double* coords, const int32_t* enodes,
                           const double* material, const int32_t* pos, const int32_t* order, const int32_t* cptr,
                           int ncol, T* vals, hipStream_t s) {
-  constexpr int WPB = 2;
-  constexpr bool kMfma = NN <= 16;  // one MFMA column tile per element
-  constexpr int WQ = 4;             // elements (wavefronts) per block of the MFMA kernel
   const int tk = prof::begin(s);
   auto launch = [&](const int32_t* ord, int begin, int count, bool atomic) {
-    if constexpr (kMfma)
-      elastic_assemble_mfma_kernel<T, NN, NG, WQ><<<div_up(count, WQ), 64 * WQ, 0, s>>>(
-          coords, enodes, material, pos, ord, begin, count, d->dN, d->w, vals, atomic);
-    else
-      elastic_assemble_kernel<NN, NG, T, WPB><<<div_up(count, WPB), 64 * WPB, 0, s>>>(
-          coords, enodes, material, pos, ord, begin, count, d->dN, d->w, vals, atomic);
+    q1_elastic_kernel<T, false><<<div_up(count, kQ1Elems), 256, 0, s>>>(
+        ElasticJob<T>{coords, enodes, material, pos, vals, 0, 0}, ord, begin, count, d->dN, d->w, atomic);
   };
   if (!order) {
     launch(nullptr, 0, n_elem, true);
@@ -921,24 +991,22 @@ static int launch_grid(const mife_element_desc* d, const int* ne, const double* 
       ? (double*)((char*)stage + ((size_t)E * ND * ND * sizeof(T) + 255) / 256 * 256)
       : nullptr;
   const int tk = prof::begin(s);
-  constexpr int WQ = 4;
-  const int grid_e = div_up(div_up(E, WQ), 8) * 8;  // a multiple of the XCD count
+  // multiples of the XCD count
+  [[maybe_unused]] const int grid_e = div_up(div_up(E, kQ2Waves), 8) * 8;
+  [[maybe_unused]] const int grid_q1 = div_up(div_up(E, kQ1Elems), 8) * 8;
   if constexpr (NC == 1) {
     if constexpr (NN == 27) {
-      q2_assemble_mfma_kernel<T, WQ><<<grid_e, 64 * WQ, 0, s>>>(coords, enodes, nullptr, coef, source, nullptr,
-                                                                nullptr, 0, (int)E, d->dN, d->N, d->w, kst,
-                                                                nullptr, false, sst, ne[0], ne[1]);
+      q2_assemble_mfma_kernel<T, true><<<grid_e, 64 * kQ2Waves, 0, s>>>(coords, enodes, nullptr, coef, source, nullptr,
+                                                                        nullptr, 0, (int)E, d->dN, d->N, d->w, kst,
+                                                                        nullptr, false, sst, ne[0], ne[1]);
     } else {
-      scalar_assemble_kernel<3, NN, NN, T, 4, true><<<grid_e, 64 * 4, 0, s>>>(coords, enodes, nullptr, coef, source,
-                                                                        nullptr, nullptr, 0, (int)E, d->dN, d->N,
-                                                                        d->w, kst, nullptr, false, sst, ne[0],
-                                                                        ne[1]);
+      q1_scalar_kernel<T, true><<<grid_q1, 256, 0, s>>>(
+          ScalarJob<T>{coords, enodes, nullptr, coef, source, nullptr, kst, nullptr, sst, ne[0], ne[1]}, nullptr, 0,
+          (int)E, d->dN, d->N, d->w, false);
     }
   } else {
-    elastic_assemble_mfma_kernel<T, NN, NN, WQ, true><<<grid_e, 64 * WQ, 0, s>>>(coords, enodes, coef, nullptr,
-                                                                                 nullptr,
-                                                                           0, (int)E, d->dN, d->w, kst, false, ne[0],
-                                                                           ne[1]);
+    q1_elastic_kernel<T, true><<<grid_q1, 256, 0, s>>>(ElasticJob<T>{coords, enodes, coef, nullptr, kst, ne[0], ne[1]},
+                                                       nullptr, 0, (int)E, d->dN, d->w, false);
   }
   constexpr int R = P * (64 / (P * P + 2 * P));
   const int runs = div_up(P * ne[0] + 1, R);
@@ -1064,9 +1132,9 @@ extern "C" int mife_assemble_elastic(const mife_element_desc* d, int n_elem, con
   hipStream_t s = (hipStream_t)stream;
   if (d->n_nodes == 8 && d->n_gauss == 8) {
     if (prec == MIFE_F64)
-      return launch_elastic<8, 8, double>(d, n_elem, coords, elem_nodes, material, pos, order, colour_ptr_host,
+      return launch_elastic<double>(d, n_elem, coords, elem_nodes, material, pos, order, colour_ptr_host,
                                           n_colours, (double*)vals, s);
-    return launch_elastic<8, 8, float>(d, n_elem, coords, elem_nodes, material, pos, order, colour_ptr_host,
+    return launch_elastic<float>(d, n_elem, coords, elem_nodes, material, pos, order, colour_ptr_host,
                                        n_colours, (float*)vals, s);
   }
   set_error("unsupported elastic element (nodes=%d, gauss=%d)", d->n_nodes, d->n_gauss);
@@ -1161,23 +1229,22 @@ extern "C" int mife_assemble_batch(const mife_element_desc* scalar_desc, const m
   MIFE_CHECK_HIP(hipStreamSynchronize(s));  // the host table may be reused at once
   const BatchJob* dj = (const BatchJob*)work;
   const BatchSeg* ds = (const BatchSeg*)((char*)work + align256(sizeof(BatchJob) * n_jobs));
-  constexpr int WPB = 4;
   const int tk = prof::begin(s);
   for (const Launch& L : launches) {
-    const int grid = std::max(1, std::min(div_up(L.total, WPB), kBatchGrid));
+    const int grid = std::max(1, std::min(div_up(L.total, kQ1Elems), kBatchGrid));
     if (L.kind == MIFE_JOB_SCALAR) {
       if (prec == MIFE_F64)
-        scalar_batch_kernel<double, WPB><<<grid, 64 * WPB, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
+        scalar_batch_kernel<double><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
                                                                    scalar_desc->dN, scalar_desc->N, scalar_desc->w);
       else
-        scalar_batch_kernel<float, WPB><<<grid, 64 * WPB, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
+        scalar_batch_kernel<float><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
                                                                   scalar_desc->dN, scalar_desc->N, scalar_desc->w);
     } else {
       if (prec == MIFE_F64)
-        elastic_batch_kernel<double, WPB><<<grid, 64 * WPB, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
+        elastic_batch_kernel<double><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
                                                                     elastic_desc->dN, elastic_desc->w);
       else
-        elastic_batch_kernel<float, WPB><<<grid, 64 * WPB, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
+        elastic_batch_kernel<float><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
                                                                    elastic_desc->dN, elastic_desc->w);
     }
   }

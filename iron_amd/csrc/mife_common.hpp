@@ -49,15 +49,26 @@ __device__ __forceinline__ double row_lane(double v) {
   return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ double lane_value(double v, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+// An eight-byte value of lane `lane`, as a scalar.
+template <typename V>
+__device__ __forceinline__ V lane_value(V v, int lane) {
+  static_assert(sizeof(V) == 8, "eight bytes");
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned int lo = __builtin_amdgcn_readlane((int)(unsigned int)u, lane);
+  const unsigned int hi = __builtin_amdgcn_readlane((int)(unsigned int)(u >> 32), lane);
+  return __builtin_bit_cast(V, ((unsigned long long)hi << 32) | lo);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float row_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 
 // Sums over aligned groups of 8 or 16 lanes, the same bits in every lane of a group.
-__device__ __forceinline__ double sum8(double v) {
-  v += row_lane<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += row_lane<0x4E>(v);   // quad_perm [2,3,0,1]
+template <typename T>
+__device__ __forceinline__ T sum8(T v) {
+  v += row_lane<0xB1>(v);         // quad_perm [1,0,3,2]
+  v += row_lane<0x4E>(v);         // quad_perm [2,3,0,1]
   return v + row_lane<0x141>(v);  // row_half_mirror
 }
 __device__ __forceinline__ double sum16(double v) {
