@@ -466,9 +466,11 @@ class Server:
         self.stats["table_builds"] += 1
         return nb.value
 
-    def _iterate(self, n_seg, nb, iters):
+    def _iterate(self, n_seg, nb, iters, mixed=True):
+        # a group without mixed requests has no replacements to look for inside a chunk
+        check = self.check_every if mixed else int(iters)
         call("mife_grouped_cg_iterate", n_seg, nb, self.max_segments, self.max_blocks, C.byref(self.pools),
-             ptr(self.b), ptr(self.x), ptr(self.vec5), ptr(self.vec6), self.rows_cap, int(iters), self.check_every,
+             ptr(self.b), ptr(self.x), ptr(self.vec5), ptr(self.vec6), self.rows_cap, int(iters), check,
              self.inner_rtol, ptr(self.table), ptr(self.state), fem._stream())
 
     def _init(self, n_seg, nb, table):
@@ -528,7 +530,7 @@ class Server:
                     self.graph = None
                     changed = False
                 tc = time.perf_counter()
-                self._run_chunk(len(active), nb)
+                self._run_chunk(len(active), nb, any(e["mixed"] for e in active))
                 self.stats["chunks"] += 1
                 self.timing["chunk"] += time.perf_counter() - tc
                 launched = True
@@ -613,13 +615,13 @@ class Server:
         self._pending.clear()
         return queue
 
-    def _run_chunk(self, n_seg, nb):
+    def _run_chunk(self, n_seg, nb, mixed=True):
         # a capture needs the structure worker idle (its allocations may synchronise
         # the device, which would invalidate the capture); only this thread submits
         # builds, so none starts during the capture
         worker_busy = any(not f.done() for f in self._pending.values())
         if not self.use_graph or (self.graph is None and worker_busy):
-            self._iterate(n_seg, nb, self.chunk)
+            self._iterate(n_seg, nb, self.chunk, mixed)
             return
         if self.graph is None:
             g = torch.cuda.CUDAGraph()
@@ -627,7 +629,7 @@ class Server:
             s.wait_stream(torch.cuda.current_stream())
             with torch.cuda.stream(s):
                 with torch.cuda.graph(g, stream=s):
-                    self._iterate(n_seg, nb, self.chunk)
+                    self._iterate(n_seg, nb, self.chunk, mixed)
             torch.cuda.current_stream().wait_stream(s)
             self.graph = g
             self.stats["graph_captures"] += 1
