@@ -565,25 +565,6 @@ __global__ void fill_kernel(int n, T* __restrict__ v, T val) {
 constexpr int kDotChunks = 8;
 constexpr int kAxpyWaves = 8;
 
-// parts[j kDotChunks + c] = V_j . w over row chunk c; block (c, j).
-__global__ __launch_bounds__(256) void gs_dots_kernel(int n, const double* __restrict__ V, size_t ldv,
-                                                      const double* __restrict__ w, double* __restrict__ parts) {
-  __shared__ double red[4];
-  const int c = blockIdx.x, j = blockIdx.y;
-  const int per = (n + kDotChunks - 1) / kDotChunks;
-  const int i1 = min(n, (c + 1) * per);
-  const double* Vj = V + (size_t)j * ldv;
-  double s0 = 0.0, s1 = 0.0;
-  int i = c * per + threadIdx.x;
-  for (; i + 256 < i1; i += 512) {
-    s0 += Vj[i] * w[i];
-    s1 += Vj[i + 256] * w[i + 256];
-  }
-  if (i < i1) s0 += Vj[i] * w[i];
-  const double t = block_sum(s0 + s1, red);
-  if (threadIdx.x == 0) parts[j * kDotChunks + c] = t;
-}
-
 // Coefficient j from its chunk partials (fixed order).
 __device__ __forceinline__ double dot_coef(const double* __restrict__ parts, int j) {
   double s = 0.0;
@@ -592,22 +573,31 @@ __device__ __forceinline__ double dot_coef(const double* __restrict__ parts, int
   return s;
 }
 
-// w -= sum_{j < m} V_j h_j with h from the dot partials hp; NORM: also the block
-// partials of the updated w.w into nparts[blockIdx.x] (blocks loop over 64-row
-// tiles).
+// The newest basis vector from the product w and its dot partials hp with the m
+// vectors so far: w scale - sum_{j < m} V_j h_j.  The basis is kept unnormalised,
+// vector j times scl[j] has norm one, and the product is that of the unnormalised
+// vector m - 1 (scale = scl[m - 1]; 1 in a refinement pass, whose w is scaled
+// already).  NORM: the result is V_m, with t = D^-1 V_m (the next product's input) and
+// the block partials of V_m.V_m in nparts[blockIdx.x]; otherwise it overwrites w.
+// Blocks loop over 64-row tiles.
 template <bool NORM>
-__global__ __launch_bounds__(64 * kAxpyWaves) void gs_axpy_kernel(int n, int m, const double* __restrict__ V,
-                                                                  size_t ldv, const double* __restrict__ hp,
+__global__ __launch_bounds__(64 * kAxpyWaves) void gs_axpy_kernel(int n, int m, double* __restrict__ V, size_t ldv,
+                                                                  const double* __restrict__ hp,
+                                                                  const double* __restrict__ scl, int scaled,
                                                                   double* __restrict__ w,
+                                                                  const double* __restrict__ dinv,
+                                                                  double* __restrict__ t,
                                                                   double* __restrict__ nparts) {
   __shared__ double hs[kMaxRestart + 1];
   __shared__ double part[kAxpyWaves][64];
   const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-  for (int j = threadIdx.x; j < m; j += blockDim.x) hs[j] = dot_coef(hp, j);
+  const double scale = scaled ? 1.0 : scl[m - 1];
+  for (int j = threadIdx.x; j < m; j += blockDim.x) hs[j] = dot_coef(hp, j) * scale * scl[j] * scl[j];
   __syncthreads();
   // wavefront q takes basis vectors [j0, j1)
   const int per = (m + kAxpyWaves - 1) / kAxpyWaves;
   const int j0 = min(m, q * per), j1 = min(m, j0 + per);
+  double* out = NORM ? V + (size_t)m * ldv : w;
   double nrm = 0.0;
   for (int r0 = blockIdx.x * 64; r0 < n; r0 += gridDim.x * 64) {
     const int row = r0 + lane;
@@ -626,81 +616,142 @@ __global__ __launch_bounds__(64 * kAxpyWaves) void gs_axpy_kernel(int n, int m, 
       double acc = 0.0;
 #pragma unroll
       for (int k = 0; k < kAxpyWaves; ++k) acc += part[k][lane];
-      const double wi = w[row] - acc;
-      w[row] = wi;
-      nrm += wi * wi;
+      const double wi = w[row] * scale - acc;
+      out[row] = wi;
+      if (NORM) {
+        t[row] = dinv[row] * wi;
+        nrm += wi * wi;
+      }
     }
     __syncthreads();
   }
   if (NORM && q == 0) {
-    const double t = wave_sum(nrm);
-    if (lane == 0) nparts[blockIdx.x] = t;
+    const double s = wave_sum(nrm);
+    if (lane == 0) nparts[blockIdx.x] = s;
   }
 }
 
 // Device state of one GMRES restart cycle.
 struct GmresCycle {
-  double hk1;  // norm of the newest basis vector before scaling (0: breakdown)
+  double hk1;  // norm of the newest basis vector (0: breakdown)
   int done;    // converged, broken down or out of iterations: the cycle stops
   int k_used;  // Hessenberg columns formed
 };
 
-// Column k of the Hessenberg matrix from the two Gram-Schmidt passes (their dot
-// partials h1, h2) and the new
-// vector's norm, the previous Givens rotations applied to it, rotation k formed
-// and g rotated; H is (m+1) x m, row-major.  The column and the rotations are
-// staged in LDS by the block, thread 0 runs the sequential rotations, and the
-// block writes the column back.  Sets done when |g[k+1]| <= tol_abs, on
-// breakdown, or when this is the last iteration allowed.
-__global__ __launch_bounds__(256) void gmres_givens_kernel(int k, int m, const double* __restrict__ h1,
-                                                           const double* __restrict__ h2,
-                                                           const double* __restrict__ nparts, int nb,
-                                                           double* __restrict__ H, double* __restrict__ cs,
-                                                           double* __restrict__ sn, double* __restrict__ g,
-                                                           GmresCycle* cy, double tol_abs, int last) {
+// A finished iteration whose Hessenberg column is still to be rotated.
+struct GmresColumn {
+  int k, m;
+  const double *h1, *h2;  // dot partials of the Gram-Schmidt pass(es)
+  const double* nparts;   // nb partials of the new vector's squared norm
+  int nb;
+  double *H, *cs, *sn, *g, *scl;
+  GmresCycle* cy;
+  double tol_abs;
+  int last;
+};
+
+// Column k of the Hessenberg matrix from the Gram-Schmidt pass(es) and the new
+// vector's norm (whose reciprocal becomes its scale), the previous Givens rotations
+// applied to it, rotation k formed and g rotated; H is (m+1) x m, row-major.  The
+// column and the rotations are staged in LDS by the block (256 threads), thread 0 runs
+// the sequential rotations, kRot of them loaded at a time, and the block writes the
+// column back.  Sets done when |g[k+1]| <= tol_abs, on breakdown, or when this is the
+// last iteration allowed.
+__device__ __forceinline__ void gmres_rotate(const GmresColumn& C) {
+  constexpr int kRot = 8;
   __shared__ double col[kMaxRestart + 1];
   __shared__ double c_s[kMaxRestart], s_s[kMaxRestart];
   __shared__ double red[4];
-  if (cy->done) return;
-  // ||w||^2 from the update's per-block partials (fixed order)
+  const int k = C.k;
+  GmresCycle* cy = C.cy;
+  const int stopped = cy->done;
+  // squared norm from the update's per-block partials (fixed order)
   double q = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) q += nparts[b];
+  for (int b = threadIdx.x; b < C.nb; b += blockDim.x) q += C.nparts[b];
   const double nrm2 = block_sum(q, red);
-  for (int j = threadIdx.x; j <= k; j += blockDim.x) col[j] = dot_coef(h1, j) + (h2 ? dot_coef(h2, j) : 0.0);
+  const double hk1 = sqrt(fmax(nrm2, 0.0));
+  if (threadIdx.x == 0 && k + 1 < C.m) C.scl[k + 1] = hk1 > 0.0 ? 1.0 / hk1 : 0.0;
+  if (stopped) return;
+  const double sk = C.scl[k];
+  for (int j = threadIdx.x; j <= k; j += blockDim.x)
+    col[j] = (dot_coef(C.h1, j) * sk + (C.h2 ? dot_coef(C.h2, j) : 0.0)) * C.scl[j];
   for (int j = threadIdx.x; j < k; j += blockDim.x) {
-    c_s[j] = cs[j];
-    s_s[j] = sn[j];
+    c_s[j] = C.cs[j];
+    s_s[j] = C.sn[j];
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    const double hk1 = sqrt(fmax(nrm2, 0.0));
-    for (int j = 0; j < k; ++j) {
-      const double a = col[j], b = col[j + 1];
-      col[j] = c_s[j] * a + s_s[j] * b;
-      col[j + 1] = -s_s[j] * a + c_s[j] * b;
+    double a = col[0];
+    int j = 0;
+    for (; j + kRot <= k; j += kRot) {
+      double b[kRot], cj[kRot], sj[kRot];
+#pragma unroll
+      for (int u = 0; u < kRot; ++u) b[u] = col[j + u + 1], cj[u] = c_s[j + u], sj[u] = s_s[j + u];
+#pragma unroll
+      for (int u = 0; u < kRot; ++u) {
+        col[j + u] = cj[u] * a + sj[u] * b[u];
+        a = -sj[u] * a + cj[u] * b[u];
+      }
     }
-    const double hkk = col[k];
-    const double den = hypot(hkk, hk1);
-    const double c = den > 0.0 ? hkk / den : 1.0, sv = den > 0.0 ? hk1 / den : 0.0;
-    cs[k] = c;
-    sn[k] = sv;
+    for (; j < k; ++j) {
+      const double b = col[j + 1];
+      col[j] = c_s[j] * a + s_s[j] * b;
+      a = -s_s[j] * a + c_s[j] * b;
+    }
+    const double den = hypot(a, hk1);
+    const double c = den > 0.0 ? a / den : 1.0, sv = den > 0.0 ? hk1 / den : 0.0;
+    C.cs[k] = c;
+    C.sn[k] = sv;
     col[k] = den;
-    const double gk = g[k];
-    g[k + 1] = -sv * gk;
-    g[k] = c * gk;
+    const double gk = C.g[k];
+    C.g[k + 1] = -sv * gk;
+    C.g[k] = c * gk;
     cy->hk1 = hk1;
     cy->k_used = k + 1;
-    if (fabs(sv * gk) <= tol_abs || hk1 == 0.0 || last) cy->done = 1;
+    if (fabs(sv * gk) <= C.tol_abs || hk1 == 0.0 || C.last) cy->done = 1;
   }
   __syncthreads();
-  for (int j = threadIdx.x; j <= k; j += blockDim.x) H[j * m + k] = col[j];
+  for (int j = threadIdx.x; j <= k; j += blockDim.x) C.H[j * C.m + k] = col[j];
+}
+
+__global__ __launch_bounds__(256) void gmres_rotate_kernel(GmresColumn C) { gmres_rotate(C); }
+
+// parts[j kDotChunks + c] = V_j . w over row chunk c; block (c, j).  PENDING: the
+// first block of the launch rotates the previous iteration's column meanwhile (GMRES
+// read one new Hessenberg column per iteration in a launch of its own, 7.4 us of which
+// the rotations' chain was most, and normalised the new vector in another, 3.9 us:
+// 53.7 us per iteration of 46,572 unknowns at restart 256, 45.5 now).
+template <bool PENDING>
+__global__ __launch_bounds__(256) void gs_dots_kernel(int n, const double* __restrict__ V, size_t ldv,
+                                                      const double* __restrict__ w, double* __restrict__ parts,
+                                                      GmresColumn C) {
+  __shared__ double red[4];
+  const int c = blockIdx.x, j = (int)blockIdx.y - (PENDING ? 1 : 0);
+  if constexpr (PENDING) {
+    if (j < 0) {
+      if (c == 0) gmres_rotate(C);
+      return;
+    }
+  }
+  const int per = (n + kDotChunks - 1) / kDotChunks;
+  const int i1 = min(n, (c + 1) * per);
+  const double* Vj = V + (size_t)j * ldv;
+  double s0 = 0.0, s1 = 0.0;
+  int i = c * per + threadIdx.x;
+  for (; i + 256 < i1; i += 512) {
+    s0 += Vj[i] * w[i];
+    s1 += Vj[i + 256] * w[i + 256];
+  }
+  if (i < i1) s0 += Vj[i] * w[i];
+  const double t = block_sum(s0 + s1, red);
+  if (threadIdx.x == 0) parts[j * kDotChunks + c] = t;
 }
 
 // Start of a restart cycle: V_0 = r / beta and t = D^-1 V_0 (the first product's
 // input), g = (beta, 0, ...), state cleared.
 __global__ void gmres_cycle_init_kernel(int n, int m, const double* __restrict__ r, double* __restrict__ V0,
                                         const double* __restrict__ dinv, double* __restrict__ t, double beta,
-                                        double* __restrict__ g, GmresCycle* cy) {
+                                        double* __restrict__ g, double* __restrict__ scl, GmresCycle* cy) {
   const int tid = blockIdx.x * blockDim.x + threadIdx.x;
   for (int i = tid; i < n; i += gridDim.x * blockDim.x) {
     const double v = r[i] / beta;
@@ -709,33 +760,20 @@ __global__ void gmres_cycle_init_kernel(int n, int m, const double* __restrict__
   }
   for (int j = tid; j <= m; j += gridDim.x * blockDim.x) g[j] = j == 0 ? beta : 0.0;
   if (tid == 0) {
+    scl[0] = 1.0;
     cy->hk1 = 0.0;
     cy->done = 0;
     cy->k_used = 0;
   }
 }
 
-// V_{k+1} = w / hk1 and t = D^-1 V_{k+1} (the next product's input) while the
-// cycle runs (nothing once it has stopped).
-__global__ void gmres_next_basis_kernel(int n, const double* __restrict__ w, double* __restrict__ v,
-                                        const double* __restrict__ dinv, double* __restrict__ t,
-                                        const GmresCycle* cy) {
-  if (cy->done) return;
-  const double a = cy->hk1 > 0.0 ? 1.0 / cy->hk1 : 0.0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const double vi = a * w[i];
-    v[i] = vi;
-    t[i] = dinv[i] * vi;
-  }
-}
-
-// x += dinv * (V y)
+// x += dinv * (V y), the basis vectors scaled by scl
 __global__ void gmres_update_kernel(int n, int m, const double* __restrict__ V, size_t ldv,
-                                    const double* __restrict__ y, const double* __restrict__ dinv,
-                                    double* __restrict__ x) {
+                                    const double* __restrict__ scl, const double* __restrict__ y,
+                                    const double* __restrict__ dinv, double* __restrict__ x) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     double s = 0.0;
-    for (int j = 0; j < m; ++j) s += V[j * ldv + i] * y[j];
+    for (int j = 0; j < m; ++j) s += V[j * ldv + i] * (scl[j] * y[j]);
     x[i] += dinv[i] * s;
   }
 }
@@ -773,78 +811,124 @@ __device__ __forceinline__ double block_fixed_sum(const double* __restrict__ par
   return block_sum(acc, red);
 }
 
+// What the rows of launch A(k) need, found while their product's loads are in flight:
+// the fixed-order sum of the nb partials of r2.z (loaded at the start of the kernel),
+// beta, and the rotation of step k-1; block 0 stores the new scalars.
+struct MinresHook {
+  static constexpr bool kActive = true;
+  MinresState* st;
+  double* red;
+  int k, nb;
+  bool done;
+  double v[2], ib, rb, phi, denom, delta, oldeps;
+  __device__ __forceinline__ MinresHook(MinresState* s, int kk, int n, double* r)
+      : st(s), red(r), k(kk), nb(n), done(false) {
+    const int i = threadIdx.x;
+    v[0] = i < nb ? s->part_b[i] : 0.0;
+    v[1] = i + 256 < nb ? s->part_b[i + 256] : 0.0;
+  }
+  __device__ __forceinline__ void sum_to(const double* parts, double a, double* out) {
+    for (int i = threadIdx.x + 512; i < nb; i += 256) a += parts[i];
+    const double s = wave_sum(a);
+    if ((threadIdx.x & 63) == 0) out[threadIdx.x >> 6] = s;
+  }
+  __device__ __forceinline__ void stage() {
+    sum_to(st->part_b, v[0] + v[1], red);
+    if (k == 0) {  // b.b
+      const double* bb = st->part_b + kRedBlocks;
+      const int i = threadIdx.x;
+      sum_to(bb, (i < nb ? bb[i] : 0.0) + (i + 256 < nb ? bb[i + 256] : 0.0), red + 4);
+    }
+  }
+  __device__ __forceinline__ void finish() {
+    MinresScalars S = st->s[k & 1];
+    const double beta = sqrt(fmax(uniform((red[0] + red[1]) + (red[2] + red[3])), 0.0));
+    if (k == 0) {
+      S.beta1 = beta;
+      S.oldb = 0.0;
+      S.phibar = beta;
+      S.cs = -1.0;
+      S.sn = 0.0;
+      S.dbar = 0.0;
+      S.epsln = 0.0;
+      S.bb = (red[4] + red[5]) + (red[6] + red[7]);
+      S.iters = 0;
+      S.done = (beta == 0.0 || S.maxit <= 0) ? 1 : 0;
+    } else {
+      oldeps = uniform(S.epsln);
+      delta = uniform(S.cs * S.dbar + S.sn * S.alfa);
+      const double gbar = S.sn * S.dbar - S.cs * S.alfa;
+      S.epsln = S.sn * beta;
+      S.dbar = -S.cs * beta;
+      const double gamma = fmax(sqrt(gbar * gbar + beta * beta), 1e-300);
+      S.cs = gbar / gamma;
+      S.sn = beta / gamma;
+      phi = uniform(S.cs * S.phibar);
+      S.phibar = S.sn * S.phibar;
+      denom = uniform(1.0 / gamma);
+      S.oldb = S.beta;
+      S.iters += 1;
+      S.done = (S.phibar <= S.tol * S.beta1 || S.iters >= S.maxit || beta == 0.0) ? 1 : 0;
+    }
+    S.beta = beta;
+    done = S.done != 0;
+    ib = uniform(beta > 0.0 ? 1.0 / beta : 0.0);
+    rb = uniform(S.oldb != 0.0 ? beta / S.oldb : 0.0);
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->s[(k + 1) & 1] = S;
+  }
+};
+
+struct MinresRow {
+  double z, r1, v, w, w2, x;
+};
+
+// Bound by the matrix stream and, at 46,572 rows, by the latency of what precedes it:
+// with the sum of the partials before the product and the rows' vectors loaded after it
+// a launch took 18.3 us (FP32 values), 17.2 now.  The product of the launch
+// that finds the iteration finished is discarded.
 template <int FMT, int L, typename TV>
 __global__ __launch_bounds__(256) void minres_a_kernel(MatArgs A, const TV* __restrict__ vals,
                                                        const double* __restrict__ z, double* __restrict__ v,
                                                        double* __restrict__ t, const double* __restrict__ r1,
-                                                       double* __restrict__ w, double* __restrict__ w1,
-                                                       double* __restrict__ w2, double* __restrict__ x,
-                                                       MinresState* st, int k, int nb) {
-  MinresScalars S = st->s[k & 1];
-  if (S.done) {  // carry the final state forward so every later launch sees it
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->s[(k + 1) & 1] = S;
+                                                       double* __restrict__ w, double* __restrict__ w2,
+                                                       double* __restrict__ x, MinresState* st, int k, int nb) {
+  // node rows (three to a lane) leave no registers for all of a row's vectors
+  constexpr bool kAll = FMT != kFmtSell3;
+  __shared__ double red[8];
+  if (st->s[k & 1].done) {  // carry the final state forward so every later launch sees it
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->s[(k + 1) & 1] = st->s[k & 1];
     return;
   }
-  const double rz = block_fixed_sum(st->part_b, nb);
-  const double beta = sqrt(fmax(rz, 0.0));
-  bool pend = false;
-  double phi = 0.0, denom = 0.0, delta = 0.0, oldeps = 0.0;
-  if (k == 0) {
-    const double bb = block_fixed_sum(st->part_b + kRedBlocks, nb);
-    S.beta1 = beta;
-    S.oldb = 0.0;
-    S.phibar = beta;
-    S.cs = -1.0;
-    S.sn = 0.0;
-    S.dbar = 0.0;
-    S.epsln = 0.0;
-    S.bb = bb;
-    S.iters = 0;
-    S.done = (beta == 0.0 || S.maxit <= 0) ? 1 : 0;
-  } else {
-    oldeps = S.epsln;
-    delta = S.cs * S.dbar + S.sn * S.alfa;
-    const double gbar = S.sn * S.dbar - S.cs * S.alfa;
-    S.epsln = S.sn * beta;
-    S.dbar = -S.cs * beta;
-    const double gamma = fmax(sqrt(gbar * gbar + beta * beta), 1e-300);
-    S.cs = gbar / gamma;
-    S.sn = beta / gamma;
-    phi = S.cs * S.phibar;
-    S.phibar = S.sn * S.phibar;
-    denom = 1.0 / gamma;
-    S.oldb = S.beta;
-    S.iters += 1;
-    S.done = (S.phibar <= S.tol * S.beta1 || S.iters >= S.maxit || beta == 0.0) ? 1 : 0;
-    pend = true;
-  }
-  S.beta = beta;
-  const bool done = S.done != 0;
-  const double ib = beta > 0.0 ? 1.0 / beta : 0.0, rb = S.oldb != 0.0 ? beta / S.oldb : 0.0;
+  MinresHook hook(st, k, nb, red);
   double m[1] = {0.0};
-  for_each_row<double, FMT, L, TV>(A, vals, done ? nullptr : z, [&](int row, double az) {
-    if (pend) {
-      const double wo = w[row], w2o = w2[row];
-      const double wn = (v[row] - oldeps * w2o - delta * wo) * denom;
-      w1[row] = w2o;
-      w2[row] = wo;
-      w[row] = wn;
-      x[row] += phi * wn;
-    }
-    if (!done) {
-      const double vi = z[row] * ib;
-      const double ti = az * ib - rb * r1[row];
-      v[row] = vi;
-      t[row] = ti;
-      m[0] += vi * ti;
-    }
-  });
-  if (!done) {
-    __shared__ double red[4];
-    double sm = block_sum(m[0], red);
-    if (threadIdx.x == 0) st->part_a[blockIdx.x] = sm;
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->s[(k + 1) & 1] = S;
+  walk_rows<double, FMT, L, TV>(
+      A, vals, z,
+      [&](int row) {
+        MinresRow o = {z[row], r1[row], 0.0, 0.0, 0.0, 0.0};
+        if (kAll && k > 0) o.v = v[row], o.w = w[row], o.w2 = w2[row], o.x = x[row];
+        return o;
+      },
+      [&](int row, double az, MinresRow o) {
+        if (!kAll && k > 0) o.v = v[row], o.w = w[row], o.w2 = w2[row], o.x = x[row];
+        if (k > 0) {
+          const double wn = (o.v - hook.oldeps * o.w2 - hook.delta * o.w) * hook.denom;
+          w2[row] = o.w;
+          w[row] = wn;
+          x[row] = o.x + hook.phi * wn;
+        }
+        if (!hook.done) {
+          const double vi = o.z * hook.ib;
+          const double ti = az * hook.ib - hook.rb * o.r1;
+          v[row] = vi;
+          t[row] = ti;
+          m[0] += vi * ti;
+        }
+      },
+      hook);
+  if (hook.done) return;
+  __shared__ double red2[4];
+  const double sm = block_sum(m[0], red2);
+  if (threadIdx.x == 0) st->part_a[blockIdx.x] = sm;
 }
 
 __global__ __launch_bounds__(256) void minres_b_kernel(int n, double* __restrict__ t, double* __restrict__ r1,
@@ -1269,7 +1353,7 @@ static void refine_layout(Work& w, int n, RefineBufs& B) {
 struct MinresBufs {
   MinresState* st;
   CgState* rs;
-  double *dinv, *b, *x, *z, *v, *t, *r1, *r2, *wv, *w1, *w2;
+  double *dinv, *b, *x, *z, *v, *t, *r1, *r2, *wv, *w2;
 };
 
 static void minres_layout(Work& w, int n, MinresBufs& B) {
@@ -1284,7 +1368,7 @@ static void minres_layout(Work& w, int n, MinresBufs& B) {
   B.r1 = w.take<double>(n);
   B.r2 = w.take<double>(n);
   B.wv = w.take<double>(n);
-  B.w1 = w.take<double>(n);
+  w.take<double>(n);  // unused; workspaces keep their size
   B.w2 = w.take<double>(n);
 }
 
@@ -1607,7 +1691,7 @@ int minres_impl(const mife_matrix* A, const TV* vals, const double* b_in, double
   MinresState* st = B.st;
   CgState* rs = B.rs;
   double *dinv = B.dinv, *b = B.b, *x = B.x, *z = B.z, *v = B.v, *t = B.t, *r1 = B.r1, *r2 = B.r2, *wv = B.wv,
-         *w1 = B.w1, *w2 = B.w2;
+         *w2 = B.w2;
   const int vg = vec_grid(n);
   const int grid = row_grid(M.a, M.a.fmt != MIFE_FMT_CSR ? 64 : M.L);
   permute_in_kernel<double><<<vg, 256, 0, s>>>(n, M.perm, b_in, b);
@@ -1615,7 +1699,6 @@ int minres_impl(const mife_matrix* A, const TV* vals, const double* b_in, double
   launch_diag_inv<double, TV>(M.a, M.stored, vals, dinv, s);
   pc_override_kernel<<<vg, 256, 0, s>>>(n, M.perm, pc_inv, dinv, 1);
   fill_kernel<double><<<vg, 256, 0, s>>>(n, v, 0.0);
-  fill_kernel<double><<<vg, 256, 0, s>>>(n, w1, 0.0);
   MIFE_DISPATCH_FMT(M.a, M.L, (minres_init_kernel<FMT_, L_, TV><<<grid, 256, 0, s>>>(M.a, vals, b, x, dinv, r1, r2,
                                                                                        z, wv, w2, st, rtol, maxit)));
   MIFE_CHECK_HIP(hipGetLastError());
@@ -1625,8 +1708,8 @@ int minres_impl(const mife_matrix* A, const TV* vals, const double* b_in, double
     for (int c = 0; c < chunk; ++c, ++k) {
       const int nb = (k == 0) ? grid : vg;
       const int tk = prof::begin(s);
-      MIFE_DISPATCH_FMT(M.a, M.L, (minres_a_kernel<FMT_, L_, TV><<<grid, 256, 0, s>>>(M.a, vals, z, v, t, r1, wv, w1,
-                                                                                        w2, x, st, k, nb)));
+      MIFE_DISPATCH_FMT(M.a, M.L, (minres_a_kernel<FMT_, L_, TV><<<grid, 256, 0, s>>>(M.a, vals, z, v, t, r1, wv, w2,
+                                                                                        x, st, k, nb)));
       prof::end(tk, s, prof::kMinresSpmv);
       minres_b_kernel<<<vg, 256, 0, s>>>(n, t, r1, r2, z, dinv, st, k, grid);
     }
@@ -1696,6 +1779,7 @@ int mife_gmres(const mife_matrix* A, const double* vals, const double* b_in, dou
   double *dinv = B.dinv, *r = B.r, *t = B.t, *wv = B.wv, *b = B.b, *x = B.x, *V = B.V;
   double *hdev = B.hdev, *ydev = B.ydev, *ndev = B.ndev, *Hdev = B.Hdev, *csdev = B.csdev, *sndev = B.sndev,
          *gdev = B.gdev;
+  double* scl = Hdev + (size_t)m * m;  // row m of H, which no column reaches
   GmresCycle* cy = B.cy;
   const size_t ldv = B.ldv;
   const int vg = vec_grid(n);
@@ -1719,8 +1803,10 @@ int mife_gmres(const mife_matrix* A, const double* vals, const double* b_in, dou
   constexpr int kChunk = 8;
   std::vector<double> H((size_t)(m + 1) * m), g(m + 2);
   while (bn > 0 && beta / bn > rtol && it < maxit) {
-    gmres_cycle_init_kernel<<<vg, 256, 0, s>>>(n, m, r, V, dinv, t, beta, gdev, cy);
+    gmres_cycle_init_kernel<<<vg, 256, 0, s>>>(n, m, r, V, dinv, t, beta, gdev, scl, cy);
     GmresCycle hc{};
+    GmresColumn col{};
+    bool pending = false;
     int k = 0;
     while (k < m) {
       const int cnt = std::min(kChunk, std::min(m - k, maxit - it));
@@ -1729,18 +1815,26 @@ int mife_gmres(const mife_matrix* A, const double* vals, const double* b_in, dou
         launch_spmv<double>(M.a, vals, t, wv, M.L, s);   // t = D^-1 V_kk (written with V_kk)
         // classical Gram-Schmidt: coefficients h, then (refinement "always") a
         // second pass with the correction y; the last update also yields the
-        // norm partials, which the rotation kernel reduces
-        gs_dots_kernel<<<dim3(kDotChunks, kk + 1), 256, 0, s>>>(n, V, ldv, wv, hdev);
+        // norm partials.  The column is rotated within the next iteration's dots
+        // (whose partials go to the other buffer), at the end of a chunk and with
+        // refinement, which needs both buffers, by a launch of its own.
+        double* h = !refine && (kk & 1) ? ydev : hdev;
+        const dim3 dots(kDotChunks, kk + 1);
+        if (pending)
+          gs_dots_kernel<true><<<dim3(kDotChunks, kk + 2), 256, 0, s>>>(n, V, ldv, wv, h, col);
+        else
+          gs_dots_kernel<false><<<dots, 256, 0, s>>>(n, V, ldv, wv, h, col);
         if (refine) {
-          gs_axpy_kernel<false><<<ag, 64 * kAxpyWaves, 0, s>>>(n, kk + 1, V, ldv, hdev, wv, nullptr);
-          gs_dots_kernel<<<dim3(kDotChunks, kk + 1), 256, 0, s>>>(n, V, ldv, wv, ydev);
-          gs_axpy_kernel<true><<<ag, 64 * kAxpyWaves, 0, s>>>(n, kk + 1, V, ldv, ydev, wv, ndev);
-        } else {
-          gs_axpy_kernel<true><<<ag, 64 * kAxpyWaves, 0, s>>>(n, kk + 1, V, ldv, hdev, wv, ndev);
+          gs_axpy_kernel<false><<<ag, 64 * kAxpyWaves, 0, s>>>(n, kk + 1, V, ldv, h, scl, 0, wv, dinv, t, ndev);
+          gs_dots_kernel<false><<<dots, 256, 0, s>>>(n, V, ldv, wv, ydev, col);
         }
-        gmres_givens_kernel<<<1, 256, 0, s>>>(kk, m, hdev, refine ? ydev : nullptr, ndev, ag, Hdev, csdev, sndev,
-                                             gdev, cy, rtol * bn, (it + c + 1 >= maxit || kk + 1 == m) ? 1 : 0);
-        gmres_next_basis_kernel<<<vg, 256, 0, s>>>(n, wv, V + (kk + 1) * ldv, dinv, t, cy);
+        gs_axpy_kernel<true><<<ag, 64 * kAxpyWaves, 0, s>>>(n, kk + 1, V, ldv, refine ? ydev : h, scl,
+                                                            refine ? 1 : 0, wv, dinv, t, ndev);
+        col = GmresColumn{kk,    m,    h,     refine ? ydev : nullptr, ndev, ag,        Hdev,
+                          csdev, sndev, gdev, scl,                     cy,   rtol * bn,
+                          (it + c + 1 >= maxit || kk + 1 == m) ? 1 : 0};
+        pending = !refine && c + 1 < cnt;
+        if (!pending) gmres_rotate_kernel<<<1, 256, 0, s>>>(col);
       }
       MIFE_CHECK_HIP(hipGetLastError());
       MIFE_CHECK_HIP(hipMemcpyAsync(&hc, cy, sizeof(GmresCycle), hipMemcpyDeviceToHost, s));
@@ -1761,7 +1855,7 @@ int mife_gmres(const mife_matrix* A, const double* vals, const double* b_in, dou
       y[i] = sum / H[(size_t)i * m + i];
     }
     MIFE_CHECK_HIP(hipMemcpyAsync(ydev, y.data(), sizeof(double) * k_used, hipMemcpyHostToDevice, s));
-    gmres_update_kernel<<<vg, 256, 0, s>>>(n, k_used, V, ldv, ydev, dinv, x);
+    gmres_update_kernel<<<vg, 256, 0, s>>>(n, k_used, V, ldv, scl, ydev, dinv, x);
     launch_residual64(M, vals, b, x, r, st, s);
     rc = read_state(st, &hs, s);
     if (rc) return rc;
