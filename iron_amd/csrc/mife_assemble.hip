@@ -1,6 +1,7 @@
 // Element integration + scatter-add into CSR values.
 //
-// One 64-lane wavefront integrates one element: lanes gather the element's
+// One 64-lane wavefront integrates one element (trilinear hexahedra: eight, further
+// down): lanes gather the element's
 // node coordinates into LDS, one lane per Gauss point forms dx/dxi, its
 // inverse and |J| (always FP64), then the lanes build the physical gradients
 // B[(g,i)][a] and contract K = B^T W B in the value precision T, and finally
