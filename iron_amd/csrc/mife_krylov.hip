@@ -936,7 +936,8 @@ __global__ __launch_bounds__(256) void minres_a_kernel(MatArgs A, const TV* __re
         }
       },
       hook);
-  if (hook.done) return;
+  // by every thread, also when the iteration is finished (a sum of zeros then): only the
+  // wavefronts that emit rows know that it is
   __shared__ double red2[4];
   const double sm = block_sum(m[0], red2);
   if (threadIdx.x == 0) st->part_a[blockIdx.x] = sm;

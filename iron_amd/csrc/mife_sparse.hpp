@@ -322,11 +322,13 @@ __device__ __forceinline__ void sell3_row_part(const MatArgs& A, const TV* __res
 
 // What a row walk does besides the rows.  pre(row) runs before the row's sum, on
 // the lane that will emit the row, and its result is handed to f: loads it issues
-// are in flight during the product.  hook.stage() and hook.finish() run once per
-// block around the walk's first barrier, after the block's first product (walks
-// without a schedule: before their rows): a block-wide sum whose operands were
-// loaded at the start of the kernel is formed there without a barrier or a wait of
-// its own.
+// are in flight during the product.  hook.stage() runs once on every wavefront of the
+// block, after its first product (walks without a schedule: before their rows), and
+// after a barrier hook.finish() runs on the wavefronts that emit rows: a block-wide sum
+// whose operands were loaded at the start of the kernel is formed there without a wait
+// of its own, and, where wavefronts share slices, at the barrier that joins their
+// parts.  What finish() leaves is for f alone: a wavefront that emits no row does not
+// have it, so no barrier may depend on it.
 // Blocks of a row walk have kWalkWaves wavefronts.
 constexpr int kWalkWaves = 4;
 
