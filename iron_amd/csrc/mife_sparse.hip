@@ -118,18 +118,21 @@ __global__ __launch_bounds__(256) void solver_rhs_kernel(int n_free, const int32
   __syncthreads();
   const int listed = count;
   for (int l = t >> 4; l < listed; l += 16) {
-    const int e = k1s[l];
+    // entries counted from the row's first one: its last may be entry 2^31 - 1
+    const int* cl = col + k0s[l];
+    const double* vl = vals + k0s[l];
+    const unsigned len = k1s[l] - k0s[l];
     double lift = 0.0;
-    for (int k = k0s[l] + sub; k < e; k += 64) {
+    for (unsigned k = sub; k < len; k += 64) {
       // every entry's value, DOF number and u, used or not: no load waits for another
       // one's test
       int j[4], fix[4];
       double kv[4], uj[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int kq = min(k + 16 * q, e - 1);
-        j[q] = col[kq];
-        kv[q] = vals[kq];
+        const unsigned kq = min(k + 16 * q, len - 1);
+        j[q] = cl[kq];
+        kv[q] = vl[kq];
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -138,7 +141,7 @@ __global__ __launch_bounds__(256) void solver_rhs_kernel(int n_free, const int32
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (k + 16 * q < e && fix[q] < 0 && fabs(uj[q]) >= ZT && fabs(kv[q]) >= ZT) lift += -1.0 * kv[q] * uj[q];
+        if (k + 16 * q < len && fix[q] < 0 && fabs(uj[q]) >= ZT && fabs(kv[q]) >= ZT) lift += -1.0 * kv[q] * uj[q];
     }
     lift = sum16(lift);
     if (sub == 0) lift_s[who[l]] = lift;
@@ -183,33 +186,40 @@ __global__ __launch_bounds__(256) void backsub_kernel(int n, const int32_t* __re
     if (rhs_fixed && rhs_fixed[row]) e = a;  // an empty row
     if (src) s = src[row];
   }
-  for (int t0 = e0; t0 < e1; t0 += kBsTile) {
-    const int k = t0 + threadIdx.x, left = e1 - k;
+  // tile ends are reached by what is left, never by adding to an entry index, which may
+  // be the last one of its type
+  for (int t0 = e0, left = e1 - e0; left > 0; left -= kBsTile) {
+    const double* vt = vals + t0;
+    const int t = threadIdx.x;
     double kv[U];
     if (iron_compat) {
 #pragma unroll
-      for (int q = 0; q < U; ++q) kv[q] = 256 * q < left ? stream_load(&vals[k + 256 * q]) : 0.0;
+      for (int q = 0; q < U; ++q) kv[q] = t + 256 * q < left ? stream_load(&vt[t + 256 * q]) : 0.0;
     } else {
+      const int32_t* ct = col + t0;
       int c[U];
 #pragma unroll
-      for (int q = 0; q < U; ++q) c[q] = 256 * q < left ? stream_load(&col[k + 256 * q]) : 0;
+      for (int q = 0; q < U; ++q) c[q] = t + 256 * q < left ? stream_load(&ct[t + 256 * q]) : 0;
 #pragma unroll
-      for (int q = 0; q < U; ++q) kv[q] = 256 * q < left ? stream_load(&vals[k + 256 * q]) : 0.0;
+      for (int q = 0; q < U; ++q) kv[q] = t + 256 * q < left ? stream_load(&vt[t + 256 * q]) : 0.0;
 #pragma unroll
       for (int q = 0; q < U; ++q) kv[q] *= u[c[q]];
     }
 #pragma unroll
-    for (int q = 0; q < U; ++q) prod[threadIdx.x + 256 * q] = kv[q];
+    for (int q = 0; q < U; ++q) prod[t + 256 * q] = kv[q];
     __syncthreads();
-    const int hi = min(e, t0 + kBsTile);
+    const int hi = min(e - t0, kBsTile), lo = max(a - t0, 0);
     if (iron_compat) {
       // equations_set_routines.F90:1806 reads the dependent value at the position
       // within the row; the correct product reads it at the column.
-      for (int j = max(a, t0) + sub; j < hi; j += 8) acc += prod[j - t0] * u[j - a];
+      for (int j = lo + sub; j < hi; j += 8) acc += prod[j] * u[j + (t0 - a)];
     } else {
-      for (int j = max(a, t0) + sub; j < hi; j += 8) acc += prod[j - t0];
+      for (int j = lo + sub; j < hi; j += 8) acc += prod[j];
     }
-    if (t0 + kBsTile < e1) __syncthreads();
+    if (left > kBsTile) {
+      t0 += kBsTile;
+      __syncthreads();
+    }
   }
   acc = sum8(acc);
   if (row < n && sub == 0) R[row] = acc - s;
