@@ -4,6 +4,7 @@
 #include "mife_sparse.hpp"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace mife {
@@ -157,27 +158,37 @@ __global__ void field_update_kernel(int n_free, const int32_t* __restrict__ free
 }
 
 // R_i = sum_k K_ik u_j - s_i for the rows whose RHS DOF is free (R_i = -s_i for
-// the others).  Bound by HBM: 12 B per entry.  A block takes kBsRows rows, whose
-// entries are one contiguous range, and reads them tile by tile with all its lanes,
-// eight entries in flight per thread, into LDS (as products K_ik u_j); eight lanes
-// per row then add the row's part of the tile.  Reading row by row with 16 lanes
-// split every load into four misaligned pieces: 75 x 83 x 67 nodes (25.9 M entries, 311
-// and 207 MB for K u and the in-row form), average of both 84 us, now 66 us; 97^3
-// nodes (57 M entries) K u 257 us, now 170 us.  Tiles of 1,024 entries, or loads one
-// tile ahead, measured 9 to 15% slower.
-constexpr int kBsRows = 32;
+// the others).  Bound by HBM: 12 B per entry (8 B in the in-row form).  A block takes ROWS
+// rows, whose entries are one contiguous range, and reads them tile by tile with all its
+// lanes, eight entries in flight per thread, into LDS (as products K_ik u_j); 256 / ROWS
+// lanes per row then add the row's part of the tile.  Walking each row with 16 lanes
+// splits every load into four misaligned pieces.  Rows walked -> tiles, matrices in turn
+// (over 1 GB of them, none in a cache): K u on 75 x 83 x 67 triquadratic nodes (62 entries
+// per row) 116 -> 78 us, on 97^3 252 -> 164 us, 90^3 trilinear nodes (26) 90 -> 67 us,
+// 97 x 33 x 33 elasticity nodes (77) 100 -> 77 us, 1001^2 plane nodes (9) 66 -> 63 us.
+// Tiles of 1,024 entries, or loads one tile ahead, measured 9 to 15% slower.
+//
+// IN_ROW: the dependent value is read at the position within the row, as
+// equations_set_routines.F90:1806 reads it (the correct product reads it at the column).
+// Rows walked -> tiles: 66 -> 60, 138 -> 129, 56 -> 45, 56 -> 54, 53 -> 41 us on the same
+// matrices.  Its values are read with plain loads: what the Infinity Cache holds of them,
+// from before or for the K u that follows, is served from there.  Plain against
+// non-temporal: both forms one after the other 125 against 136 us (75 x 83 x 67) and 274
+// against 290 us (97^3); this form alone 60 against 56 and 129 against 120 us; this form
+// again and again on one 154 MB matrix 37 against 42 us.
 constexpr int kBsTile = 2048;
+constexpr int kBsFewRows = 16384;
 
+template <int ROWS, bool IN_ROW>
 __global__ __launch_bounds__(256) void backsub_kernel(int n, const int32_t* __restrict__ row_ptr,
                                                       const int32_t* __restrict__ col,
                                                       const double* __restrict__ vals, const double* __restrict__ u,
                                                       const double* __restrict__ src,
-                                                      const uint8_t* __restrict__ rhs_fixed, int iron_compat,
-                                                      double* __restrict__ R) {
+                                                      const uint8_t* __restrict__ rhs_fixed, double* __restrict__ R) {
   __shared__ double prod[kBsTile];
-  constexpr int U = kBsTile / 256;
-  const int r0 = blockIdx.x * kBsRows, row = r0 + (threadIdx.x >> 3), sub = threadIdx.x & 7;
-  const int e0 = row_ptr[r0], e1 = row_ptr[min(r0 + kBsRows, n)];
+  constexpr int U = kBsTile / 256, L = 256 / ROWS;
+  const int r0 = blockIdx.x * ROWS, row = r0 + threadIdx.x / L, sub = threadIdx.x % L;
+  const int e0 = row_ptr[r0], e1 = row_ptr[min(r0 + ROWS, n)];
   int a = 0, e = 0;
   double s = 0.0, acc = 0.0;
   if (row < n) {
@@ -189,39 +200,33 @@ __global__ __launch_bounds__(256) void backsub_kernel(int n, const int32_t* __re
   // tile ends are reached by what is left, never by adding to an entry index, which may
   // be the last one of its type
   for (int t0 = e0, left = e1 - e0; left > 0; left -= kBsTile) {
-    const double* vt = vals + t0;
-    const int t = threadIdx.x;
+    const double* vt = vals + t0 + threadIdx.x;
+    const int rest = left - (int)threadIdx.x;
     double kv[U];
-    if (iron_compat) {
+    if constexpr (IN_ROW) {
 #pragma unroll
-      for (int q = 0; q < U; ++q) kv[q] = t + 256 * q < left ? stream_load(&vt[t + 256 * q]) : 0.0;
+      for (int q = 0; q < U; ++q) kv[q] = 256 * q < rest ? vt[256 * q] : 0.0;
     } else {
-      const int32_t* ct = col + t0;
+      const int32_t* ct = col + t0 + threadIdx.x;
       int c[U];
 #pragma unroll
-      for (int q = 0; q < U; ++q) c[q] = t + 256 * q < left ? stream_load(&ct[t + 256 * q]) : 0;
+      for (int q = 0; q < U; ++q) c[q] = 256 * q < rest ? stream_load(ct + 256 * q) : 0;
 #pragma unroll
-      for (int q = 0; q < U; ++q) kv[q] = t + 256 * q < left ? stream_load(&vt[t + 256 * q]) : 0.0;
+      for (int q = 0; q < U; ++q) kv[q] = 256 * q < rest ? stream_load(vt + 256 * q) : 0.0;
 #pragma unroll
       for (int q = 0; q < U; ++q) kv[q] *= u[c[q]];
     }
 #pragma unroll
-    for (int q = 0; q < U; ++q) prod[t + 256 * q] = kv[q];
+    for (int q = 0; q < U; ++q) prod[threadIdx.x + 256 * q] = kv[q];
     __syncthreads();
-    const int hi = min(e - t0, kBsTile), lo = max(a - t0, 0);
-    if (iron_compat) {
-      // equations_set_routines.F90:1806 reads the dependent value at the position
-      // within the row; the correct product reads it at the column.
-      for (int j = lo + sub; j < hi; j += 8) acc += prod[j] * u[j + (t0 - a)];
-    } else {
-      for (int j = lo + sub; j < hi; j += 8) acc += prod[j];
-    }
+    const int hi = left > kBsTile ? min(e, t0 + kBsTile) : e;
+    for (int j = max(a, t0) - t0 + sub; j < hi - t0; j += L) acc += IN_ROW ? prod[j] * u[j + (t0 - a)] : prod[j];
     if (left > kBsTile) {
       t0 += kBsTile;
       __syncthreads();
     }
   }
-  acc = sum8(acc);
+  acc = L == 8 ? sum8(acc) : sum16(acc);
   if (row < n && sub == 0) R[row] = acc - s;
 }
 
@@ -461,7 +466,21 @@ int mife_backsubstitute(int n, const int32_t* row_ptr, const int32_t* col, const
                         const double* src, const uint8_t* rhs_fixed, int iron_compat, double* R, void* stream) {
   if (n == 0) return MIFE_OK;  // empty arrays may be passed as NULL
   MIFE_REQUIRE(row_ptr && col && vals && u && R, MIFE_ERR_POINTER_IS_NULL, "null pointer argument");
-  backsub_kernel<<<div_up(n, kBsRows), 256, 0, (hipStream_t)stream>>>(n, row_ptr, col, vals, u, src, rhs_fixed, iron_compat, R);
+  hipStream_t s = (hipStream_t)stream;
+  auto go = [&](auto rows) {
+    constexpr int ROWS = decltype(rows)::value;
+    const int grid = div_up(n, ROWS);
+    if (iron_compat)
+      backsub_kernel<ROWS, true><<<grid, 256, 0, s>>>(n, row_ptr, col, vals, u, src, rhs_fixed, R);
+    else
+      backsub_kernel<ROWS, false><<<grid, 256, 0, s>>>(n, row_ptr, col, vals, u, src, rhs_fixed, R);
+  };
+  // Up to 16,384 rows, 32 to a block leave the chip with at most 512 blocks, a third of
+  // which walk two tiles one after the other (15,625 triquadratic rows: 10.6 us, 8.2 with
+  // 16 rows to a block); beyond, 16 rows fill too little of a tile (90^3 trilinear nodes
+  // 95 us against 67, 75 x 83 x 67 triquadratic ones 85 against 78).
+  if (n <= kBsFewRows) go(std::integral_constant<int, 16>{});
+  else go(std::integral_constant<int, 32>{});
   MIFE_CHECK_HIP(hipGetLastError());
   return MIFE_OK;
 }

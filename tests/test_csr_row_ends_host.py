@@ -38,20 +38,28 @@ int main(int, char** argv) {
   return 0;
 }
 """
-BACKSUB = """emu::launch((n + kBsRows - 1) / kBsRows, 256, [&] {
-    backsub_kernel(n, rp.data(), colp, valp, u.data(), src.data(), nullptr, compat, R.data());
-  });"""
+BACKSUB = """const int rows = std::atoi(argv[4]);
+  auto back = [&](auto r, auto c) {
+    constexpr int ROWS = decltype(r)::value;
+    emu::launch((n + ROWS - 1) / ROWS, 256, [&] {
+      backsub_kernel<ROWS, decltype(c)::value>(n, rp.data(), colp, valp, u.data(), src.data(), nullptr, R.data());
+    });
+  };
+  auto pick = [&](auto r) { compat ? back(r, std::true_type{}) : back(r, std::false_type{}); };
+  if (rows == 16) pick(std::integral_constant<int, 16>{});
+  else pick(std::integral_constant<int, 32>{});"""
 
 
 @pytest.fixture(scope="module")
 def rows(tmp_path_factory):
-    parts = ["kRhsRows", "solver_rhs_kernel", "kBsRows", "kBsTile", "backsub_kernel"]
+    parts = ["kRhsRows", "solver_rhs_kernel", "kBsTile", "backsub_kernel"]
     source = '#include "mife_sparse.hpp"\nnamespace mife {\n' + "".join(definition("mife_sparse.hip", p) for p in parts)
     return build(tmp_path_factory.mktemp("rows"), source + "}\n", MAIN.replace("BACKSUB", BACKSUB), "-ftrapv")
 
 
 @pytest.mark.parametrize("compat", [0, 1])
+@pytest.mark.parametrize("block_rows", [16, 32])
 @pytest.mark.parametrize("n,len_", [(1, 5), (3, 70), (33, 61), (40, 130), (2, 5000)])
-def test_rows_at_the_end_of_the_index_range(rows, n, len_, compat):
-    err, = run(rows, n, len_, compat, timeout=20)
+def test_rows_at_the_end_of_the_index_range(rows, n, len_, block_rows, compat):
+    err, = run(rows, n, len_, compat, block_rows, timeout=20)
     assert err <= 1e-15 * (len_ + 2) * (len_ + n)  # rows of len_ products below 1

@@ -64,3 +64,27 @@ def test_backsubstitution_and_rhs_rows(n, kind):
         want = (src + rhs + np.bincount(rows, prod, n))[free]
         lim = EPS * ((np.maximum(lengths, 1) + 3) * (np.bincount(rows, np.abs(prod), n) + np.abs(src) + np.abs(rhs)))[free]
         assert np.all(np.abs(b.cpu().numpy() - want) <= lim)
+
+
+@pytest.mark.parametrize("n", [16383, 16384, 16385, 40001])
+def test_backsubstitution_rows_per_block(n):
+    """Row counts about the one from which a block takes 32 rows instead of 16; rows of 0 to
+    140 entries, so that blocks hold less than a tile, about one and more than two."""
+    from iron_amd import _lib
+    print(f"case n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    lengths = np.where(np.arange(n) // 500 % 2 == 0, rng.integers(0, 30, n), rng.integers(50, 141, n))
+    rp = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    rows = np.repeat(np.arange(n), lengths)
+    inrow = np.arange(rp[-1]) - rp[rows]
+    col = ((rows + 17 * inrow) % n).astype(np.int32)
+    vals, u, src = rng.standard_normal(rp[-1]), rng.standard_normal(n), rng.standard_normal(n)
+    fixed = (rng.random(n) < 0.25).astype(np.uint8)
+    d = [_dev(a) for a in (rp, col, vals, u, src, fixed)]
+    R = torch.empty(n, dtype=torch.float64, device="cuda")
+    for compat in (0, 1):
+        _lib.call("mife_backsubstitute", n, *[_lib.ptr(t) for t in d], compat, _lib.ptr(R), None)
+        prod = np.where(fixed[rows] != 0, 0.0, vals * u[inrow if compat else col])
+        want = np.bincount(rows, prod, n) - src
+        lim = EPS * (lengths + 3) * (np.bincount(rows, np.abs(prod), n) + np.abs(src))
+        assert np.all(np.abs(R.cpu().numpy() - want) <= lim)
