@@ -772,7 +772,7 @@ int mife_grouped_setup(const mife_segment* segs_host, int n_seg, int max_segment
     // sizes are not in the table, so trilinear rows are assumed (a wrong guess costs
     // cache hits, nothing else)
     const double bytes = 27.0 * S.n * (S.format == MIFE_FMT_SELL3 ? 24.7 : 10.0);
-    const int keep = kept + bytes <= kCacheBytes ? 1 : 0;
+    const int keep = kept + bytes <= kKeepMost ? 1 : 0;
     if (keep) kept += bytes;
     const int p0 = nb, p1 = nb + std::max(1, div_up(units, per));
     int r0 = 0;

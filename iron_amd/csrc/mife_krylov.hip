@@ -1074,7 +1074,8 @@ struct Mat {
   bool graphs = true;  // CG chunks may replay cached HIP graphs (not without allocation)
 };
 
-static int make_mat(const mife_matrix* A, Mat* m) {
+// `row_bytes`: bytes per row of the vectors that an iteration reads.
+static int make_mat(const mife_matrix* A, double row_bytes, Mat* m) {
   MIFE_REQUIRE(A && A->ptr && A->col, MIFE_ERR_POINTER_IS_NULL, "null matrix");
   MIFE_REQUIRE(A->format == MIFE_FMT_CSR || A->format == MIFE_FMT_SELL || A->format == MIFE_FMT_SELL3, MIFE_ERR_ARG,
                "invalid matrix format");
@@ -1085,7 +1086,7 @@ static int make_mat(const mife_matrix* A, Mat* m) {
                "SELL3 matrix needs perm, n = 3 x node rows, n_slices = ceil(n/192) and col_base");
   MIFE_REQUIRE(!A->slice_order || ((uintptr_t)A->slice_order & 15) == 0, MIFE_ERR_ARG,
                "slice_order must be 16-byte aligned");
-  m->a = mat_args(A);
+  m->a = mat_args(A, row_bytes * A->n);
   m->perm = A->format != MIFE_FMT_CSR ? A->perm : nullptr;
   m->L = spmv_lanes(A->nnz, A->n);
   m->stored = A->nnz;
@@ -1481,7 +1482,7 @@ static int cg_entry(bool graphs, const mife_matrix* A, const void* vals, const v
   MIFE_REQUIRE(prec == MIFE_F64 || prec == MIFE_F32, MIFE_ERR_ARG, "invalid precision %d", prec);
   MIFE_REQUIRE(maxit >= 0 && rtol >= 0.0, MIFE_ERR_ARG, "invalid CG arguments");
   Mat M;
-  int rc = make_mat(A, &M);
+  int rc = make_mat(A, 6.0 * (prec == MIFE_F64 ? 8 : 4), &M);
   M.graphs = graphs;  // graph instantiation may allocate
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
@@ -1602,7 +1603,7 @@ int mife_refine(const mife_matrix* A, const double* vals64, const float* vals32,
   MIFE_REQUIRE(vals64 && vals32 && b_in && x_io && work, MIFE_ERR_POINTER_IS_NULL, "null pointer argument");
   MIFE_REQUIRE(rtol > 0.0 && inner_rtol > 0.0 && inner_rtol < 1.0 && maxit > 0, MIFE_ERR_ARG, "invalid arguments");
   Mat M;
-  int rc = make_mat(A, &M);
+  int rc = make_mat(A, 6.0 * 4, &M);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const int n = M.a.n;
@@ -1696,7 +1697,7 @@ template <typename TV>
 int minres_impl(const mife_matrix* A, const TV* vals, const double* b_in, double* x_io, const double* pc_inv,
                 double rtol, int maxit, void* work, size_t work_bytes, int* iters, double* relres, void* stream) {
   Mat M;
-  int rc = make_mat(A, &M);
+  int rc = make_mat(A, 9.0 * 8, &M);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const int n = M.a.n;
@@ -1781,7 +1782,7 @@ int mife_gmres(const mife_matrix* A, const double* vals, const double* b_in, dou
   MIFE_REQUIRE(vals && b_in && x_io && work, MIFE_ERR_POINTER_IS_NULL, "null pointer argument");
   MIFE_REQUIRE(restart >= 1 && restart <= kMaxRestart && rtol > 0.0, MIFE_ERR_ARG, "invalid GMRES arguments");
   Mat M;
-  int rc = make_mat(A, &M);
+  int rc = make_mat(A, (restart + 5.0) * 8, &M);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   const int n = M.a.n;

@@ -57,17 +57,23 @@ struct MatArgs {
 
 // Sixteenths of a matrix of `bytes` (values and columns) that repeated products
 // read with plain loads, which the Infinity Cache keeps between products; the
-// other slices' non-temporal loads pass it by.  A matrix within kCacheBytes is
-// kept whole.  Measured: FP64 CG on a 96x32x32 elasticity system (200 MB of node
-// blocks) 73.4 ms all non-temporal, 62.3 ms kept whole; GMRES on a 12^3 Q2/Q1
-// Newton matrix (89 MB) 59.8 -> 53.9 ms, MINRES on its FP32 values 45.8 -> 39.0 ms;
-// a 326 MB FP32 matrix (48^3 triquadratic diffusion, whole pass) 41.3 ms all
-// non-temporal, 44.9 ms all plain (it evicts itself), 37.4 ms with 10 sixteenths
-// kept.  Kept bytes of 180 to 220 MB measured within 0.2% of each other there, 140
-// and 240 MB 1% slower.
-constexpr double kCacheBytes = 2.1e8;
-inline int keep_sixteenths(double bytes) {
-  return bytes <= kCacheBytes ? 16 : (int)(16.0 * kCacheBytes / bytes);
+// other slices' non-temporal loads pass it by.  `beside`: bytes of the vectors that an
+// iteration reads as well (a Krylov basis among them), which have the first claim; the
+// matrix gets what they leave of kCacheBytes, at most kKeepMost.  A matrix within that
+// is kept whole.  Measured, nothing kept -> kept: FP64 CG on a 96x32x32 elasticity system
+// (200 MB of node blocks) 73.4 -> 62.3 ms; GMRES on a 12^3 Q2/Q1 Newton matrix (89 MB)
+// 59.8 -> 53.9 ms, MINRES on its FP32 values 45.8 -> 39.0 ms; a 326 MB FP32 matrix (48^3
+// triquadratic diffusion, whole pass) 41.3 ms, 44.9 ms all plain (it evicts itself),
+// 37.4 ms with 10 sixteenths kept (180 to 220 MB within 0.2% of each other there, 140 and
+// 240 MB 1% slower).  Nothing, what the vectors leave, and 210 MB whatever the vectors
+// take, us per iteration: FP64 CG on 1.0 M trilinear rows (49 MB of vectors) 93.0 / 80.3 /
+// 82.1, on 4.1 M rows (199 MB) 320 / 320 / 327, on 8.1 M rows 698 / 698 / 718; GMRES(30) on
+// 0.9 M triquadratic rows (224 MB of basis) 232 / 232 / 264, on 0.7 M trilinear rows (179 MB)
+// 134 / 132 / 154, GMRES(100) on 0.12 M rows (93 MB) 50.6 / 45.0 / 45.0.
+constexpr double kCacheBytes = 2.3e8, kKeepMost = 2.1e8;
+inline int keep_sixteenths(double bytes, double beside) {
+  const double room = std::min(kKeepMost, kCacheBytes - beside);
+  return bytes <= room ? 16 : (int)(16.0 * std::max(room, 0.0) / bytes);
 }
 
 // Shape of a SELL3 descriptor: three rows per node row, ceil(node rows / 64)
@@ -80,7 +86,8 @@ inline bool sell3_shape_ok(const mife_matrix* A) {
 // the chip on small matrices (long rows, few slices), one per slice on large.
 inline int sell_split(int n_slices) { return n_slices < 4096 ? 4 : (n_slices < 65536 ? 2 : 1); }
 
-inline MatArgs mat_args(const mife_matrix* A) {
+// `beside`: what an iteration reads besides the matrix (keep_sixteenths).
+inline MatArgs mat_args(const mife_matrix* A, double beside = 0.0) {
   const bool sell3 = A->format == MIFE_FMT_SELL3;
   const bool sell = A->format == MIFE_FMT_SELL || sell3;
   const bool c16 = sell && A->col_base != nullptr;
@@ -89,8 +96,8 @@ inline MatArgs mat_args(const mife_matrix* A) {
   const double cb = sell3 ? 2.0 / 9.0 : (c16 ? 2.0 : 4.0);
   return MatArgs{A->n, sell3 ? kFmtSell3 : (c16 ? kFmtSell16 : A->format), A->ptr, A->col, A->n_slices,
                  c16 ? A->col_base : nullptr, sched ? A->slice_order : nullptr, sched ? A->order_span : 0,
-                 sched ? sell_split(A->n_slices) : 1, keep_sixteenths((8.0 + cb) * (double)A->nnz),
-                 keep_sixteenths((4.0 + cb) * (double)A->nnz)};
+                 sched ? sell_split(A->n_slices) : 1, keep_sixteenths((8.0 + cb) * (double)A->nnz, beside),
+                 keep_sixteenths((4.0 + cb) * (double)A->nnz, beside)};
 }
 
 // A matrix that is read once (a residual between other products): nothing kept.
