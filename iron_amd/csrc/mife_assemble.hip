@@ -13,6 +13,7 @@
 #include "mife_profile.hpp"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace mife {
@@ -53,24 +54,33 @@ __device__ __forceinline__ void add_value(T* p, T v, bool atomic) {
   else *p += v;
 }
 
-// N entries of one element into the CSR values (p < 0: none).  They are distinct
-// entries and no other element of the launch touches them (atomic: they may), so every
-// value is loaded before the first is stored: one round trip instead of N (a 23 x 19 x 21
+// N values into the CSR (no address: none).  They are distinct entries and no other
+// element of the launch touches them (atomic: they may), so every old value is loaded
+// before the first sum is stored: one round trip instead of N (a 23 x 19 x 21
 // triquadratic mesh, eight colour launches: 219 -> 180 us).
 template <typename T, int N>
-__device__ __forceinline__ void add_values(T* __restrict__ vals, const int (&p)[N], const T (&v)[N], bool atomic) {
+__device__ __forceinline__ void add_values(T* const (&at)[N], const T (&v)[N], bool atomic) {
   if (atomic) {
 #pragma unroll
     for (int k = 0; k < N; ++k)
-      if (p[k] >= 0) atomicAdd(&vals[p[k]], v[k]);
+      if (at[k]) atomicAdd(at[k], v[k]);
     return;
   }
   T old[N];
 #pragma unroll
-  for (int k = 0; k < N; ++k) old[k] = p[k] >= 0 ? vals[p[k]] : (T)0;
+  for (int k = 0; k < N; ++k) old[k] = at[k] ? *at[k] : (T)0;
 #pragma unroll
   for (int k = 0; k < N; ++k)
-    if (p[k] >= 0) vals[p[k]] = old[k] + v[k];
+    if (at[k]) *at[k] = old[k] + v[k];
+}
+
+// As above for entries p of one CSR (p < 0: none).
+template <typename T, int N>
+__device__ __forceinline__ void add_values(T* __restrict__ vals, const int (&p)[N], const T (&v)[N], bool atomic) {
+  T* at[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) at[k] = p[k] >= 0 ? vals + p[k] : nullptr;
+  add_values(at, v, atomic);
 }
 
 // Stage layout of a structured (grid) assembly.  With row m = (c, a), column
@@ -259,25 +269,27 @@ __global__ __launch_bounds__(64 * WPB) void scalar_assemble_kernel(
 // its inverse and the point's physical gradients in registers, and the eight points'
 // contributions to an entry meet by DPP inside the element's eight lanes.  With one
 // element per wavefront only 16 of 64 lanes formed geometry, and the sums read 72 LDS
-// values per entry.  All forms (structured, coloured, batched) run this code, with
-// every multiply-add written out, so their sums agree bit for bit.
-constexpr int kQ1Elems = 32;  // elements per block of 256 threads
-
+// values per entry.  In launches of few elements G = 8 such groups of lanes share an
+// element, a row of its matrix each.  All forms (structured, coloured, batched; whatever
+// G) run this code, with every multiply-add written out, so their sums agree bit for bit.
+// E elements to a block of 8 E G threads.
+template <int E>
 struct Q1Tables {
   double dN[8 * 8 * 3];
-  double X[kQ1Elems][8][3];
+  double X[E][8][3];
 };
 
 // Geometry of lane's (element, Gauss point q): ji[j][i] = dxi_j/dx_i, and |J| w_q.
 // Holds two block barriers.
-__device__ __forceinline__ double q1_geometry(Q1Tables& S, const double* __restrict__ coords,
+template <int E, int G = 1>
+__device__ __forceinline__ double q1_geometry(Q1Tables<E>& S, const double* __restrict__ coords,
                                               const int32_t* __restrict__ enodes, long long e, bool active,
                                               const double* __restrict__ dN, const double* __restrict__ w,
                                               double (&ji)[3][3]) {
-  const int el = threadIdx.x >> 3, q = threadIdx.x & 7;
+  const int el = threadIdx.x / (8 * G), q = threadIdx.x & 7;
   __syncthreads();  // the tables of an earlier pass are done with
-  if (threadIdx.x < 8 * 8 * 3) S.dN[threadIdx.x] = dN[threadIdx.x];
-  if (active) {
+  for (int t = threadIdx.x; t < 8 * 8 * 3; t += 8 * E * G) S.dN[t] = dN[t];
+  if (active && (threadIdx.x >> 3) % G == 0) {
     const long long node = enodes[e * 8 + q];
 #pragma unroll
     for (int d = 0; d < 3; ++d) S.X[el][q][d] = coords[node * 3 + d];
@@ -296,63 +308,77 @@ __device__ __forceinline__ double q1_geometry(Q1Tables& S, const double* __restr
   return fabs(det) * w[q];
 }
 
-// One scalar element per eight lanes (e and J are the eight lanes' own); every thread
-// of the block calls it.
-template <typename T, bool GRID>
+// One scalar element per 8 G lanes (e and J are those lanes' own); every thread of the
+// block calls it.
+template <typename T, bool GRID, int E, int G>
 __device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, long long e, bool active,
                                                    const double* __restrict__ dN, const double* __restrict__ N,
                                                    const double* __restrict__ w, bool atomic) {
 #pragma clang fp contract(off)
   using GS = GridStripe<8, 1>;
-  __shared__ Q1Tables S;
-  __shared__ double rw[kQ1Elems][8];
-  __shared__ T sK[kQ1Elems * 64];
-  __shared__ long long sbase[kQ1Elems];
-  const int el = threadIdx.x >> 3, q = threadIdx.x & 7;
+  __shared__ Q1Tables<E> S;
+  __shared__ double rw[E][8];
+  __shared__ T sK[E * 64];
+  __shared__ long long sbase[E];
+  const int el = threadIdx.x / (8 * G), q = threadIdx.x & 7, g = (threadIdx.x >> 3) % G;
   double ji[3][3];
-  const double rwg = q1_geometry(S, J.coords, J.enodes, e, active, dN, w, ji);
+  const double rwg = q1_geometry<E, G>(S, J.coords, J.enodes, e, active, dN, w, ji);
   const double ke = (active && J.kappa) ? J.kappa[e] : 1.0;
   const T W = (T)(rwg * ke);
-  T B[8][3];
-#pragma unroll
-  for (int a = 0; a < 8; ++a) {
+  auto gradient = [&](int a, T (&b)[3]) {
     const double* d = &S.dN[(q * 8 + a) * 3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) B[a][i] = (T)fma(d[0], ji[0][i], fma(d[1], ji[1][i], d[2] * ji[2][i]));
-  }
+    for (int i = 0; i < 3; ++i) b[i] = (T)fma(d[0], ji[0][i], fma(d[1], ji[1][i], d[2] * ji[2][i]));
+  };
+  T B[8][3];
+#pragma unroll
+  for (int a = 0; a < 8; ++a) gradient(a, B[a]);
   rw[el][q] = rwg;
-  int t = 0;
-#pragma unroll
-  for (int m = 0; m < 8; ++m) {
-    const T b0 = W * B[m][0], b1 = W * B[m][1], b2 = W * B[m][2];
-#pragma unroll
-    for (int n = m; n < 8; ++n, ++t) {
-      const T v = sum8(fma(b0, B[n][0], fma(b1, B[n][1], b2 * B[n][2])));
-      if (q == (t & 7)) {  // entry t of the upper triangle, and its transpose
-        sK[GRID ? GS::slot(m, n, el, kQ1Elems) : el * 64 + m * 8 + n] = v;
-        sK[GRID ? GS::slot(n, m, el, kQ1Elems) : el * 64 + n * 8 + m] = v;
-      }
+  auto entry = [&](int m, int n, const T (&bm)[3], bool mine) {  // and its transpose
+    const T v = sum8(fma(W * bm[0], B[n][0], fma(W * bm[1], B[n][1], W * bm[2] * B[n][2])));
+    if (mine) {
+      sK[GRID ? GS::slot(m, n, el, E) : el * 64 + m * 8 + n] = v;
+      sK[GRID ? GS::slot(n, m, el, E) : el * 64 + n * 8 + m] = v;
     }
+  };
+  if constexpr (G == 8) {  // row g of the upper triangle
+    T bg[3];
+    gradient(g, bg);
+#pragma unroll
+    for (int n = 0; n < 8; ++n) entry(g, n, bg, n >= g && q == n);
+  } else {  // all of it, entry t in lane t % 8
+    int t = 0;
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+      for (int n = m; n < 8; ++n, ++t) entry(m, n, B[m], q == (t & 7));
   }
-  if (GRID && q == 0) sbase[el] = active ? GS::base(e, J.gnx, J.gny) : -1;
+  if (GRID && q == 0 && g == 0) sbase[el] = active ? GS::base(e, J.gnx, J.gny) : -1;
   __syncthreads();
   if constexpr (GRID) {
-    GS::template store<T, kQ1Elems>(sK, sbase, J.gnx, J.vals);
-  } else if (active) {
-    const int32_t* pe = J.pos + e * 64 + q * 8;
-    int p[8];
-    T v[8];
+    GS::template store<T, E>(sK, sbase, J.gnx, J.vals);
+  } else {
+    // the wavefront's elements one by one, a lane per entry: the lanes of a store lie in
+    // eight rows (a row per lane instead, in eight elements at once, touched 64 lines:
+    // 61 x 47 x 53 elements, atomic, 283 us FP64 and 306 us FP32; 159 and 122 us so)
+    constexpr int N = 8 / G;
+    const int lane = threadIdx.x & 63, el0 = (threadIdx.x >> 6) * N;
+    T* at[N];
+    T v[N];
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      p[n] = pe[n];
-      v[n] = sK[el * 64 + q * 8 + n];
+    for (int i = 0; i < N; ++i) {
+      at[i] = nullptr;
+      if (__builtin_amdgcn_readlane((int)active, 8 * i)) {
+        at[i] = lane_value(J.vals, 8 * i) + lane_value(J.pos, 8 * i)[lane_value(e, 8 * i) * 64 + lane];
+        v[i] = sK[(el0 + i) * 64 + lane];
+      }
     }
-    add_values(J.vals, p, v, atomic);
+    add_values(at, v, atomic);
   }
-  if (active && J.source && (J.svec || J.sstage)) {
+  if (active && g == 0 && J.source && (J.svec || J.sstage)) {
     double s = 0.0;
 #pragma unroll
-    for (int g = 0; g < 8; ++g) s = fma(N[g * 8 + q], rw[el][g], s);
+    for (int p = 0; p < 8; ++p) s = fma(N[p * 8 + q], rw[el][p], s);
     s = s * J.source[e];
     if (J.sstage)
       J.sstage[e * 8 + q] = s;
@@ -363,17 +389,17 @@ __device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, long l
 
 // Measured on 61 x 47 x 53 elements with moved nodes, FP64, structured: 187 us with
 // one element per wavefront, 55 us now (78 MB of element matrices stored).
-template <typename T, bool GRID>
-__global__ __launch_bounds__(256) void q1_scalar_kernel(ScalarJob<T> J, const int32_t* __restrict__ order,
+template <typename T, bool GRID, int E, int G>
+__global__ __launch_bounds__(8 * E * G) void q1_scalar_kernel(ScalarJob<T> J, const int32_t* __restrict__ order,
                                                         int elem_begin, int elem_count,
                                                         const double* __restrict__ dN, const double* __restrict__ N,
                                                         const double* __restrict__ w, bool atomic) {
   const int blk = GRID ? GridStripe<8, 1>::block(J.gnx) : (int)blockIdx.x;
-  const int idx = blk * kQ1Elems + (threadIdx.x >> 3);
+  const int idx = blk * E + (threadIdx.x / (8 * G));
   const bool active = idx < elem_count;
   long long e = 0;
   if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
-  q1_scalar_elements<T, GRID>(J, e, active, dN, N, w, atomic);
+  q1_scalar_elements<T, GRID, E, G>(J, e, active, dN, N, w, atomic);
 }
 
 // ------------------------------------------------ triquadratic, on MFMA
@@ -531,20 +557,21 @@ struct ElasticJob {
   int gnx, gny;  // GRID: elements in x and y (GridStripe layout)
 };
 
-// Element 4 i + w of a block belongs to wavefront w (lanes 8 i .. 8 i + 7 hold its
+// Element 4 i + w of a block belongs to wavefront w (lanes 8 i .. 8 i + 7, i < turns, hold its
 // number and arrays): in turn i the four wavefronts take consecutive elements, whose
 // entries leave through LDS in runs of 16 values.  Half of the gradients are in LDS
 // at a time, which keeps two blocks on a CU.
+constexpr int kElasticElems = 32;  // at most, in a block of 256 threads (4 per turn)
 __device__ __forceinline__ int q1_elastic_slot() { return 4 * ((threadIdx.x & 63) >> 3) + (threadIdx.x >> 6); }
 
 template <typename T, bool GRID>
-__device__ __forceinline__ void q1_elastic_elements(const ElasticJob<T>& J, long long e, bool active,
+__device__ __forceinline__ void q1_elastic_elements(const ElasticJob<T>& J, long long e, bool active, int turns,
                                                     const double* __restrict__ dN, const double* __restrict__ w,
                                                     bool atomic) {
 #pragma clang fp contract(off)
   using GS = GridStripe<8, 3>;
-  constexpr int kWaves = kQ1Elems / 8, kHalf = 4, kRun = kWaves * GS::B2;
-  __shared__ Q1Tables S;
+  constexpr int kWaves = kElasticElems / 8, kHalf = 4, kRun = kWaves * GS::B2;
+  __shared__ Q1Tables<kElasticElems> S;
   __shared__ T sB[kWaves][kHalf][8][8][3];
   __shared__ T sW[kWaves][8][8];
   __shared__ T sC[kWaves][8][15];  // diagC[3][3], then (Ca, Cb) of the pairs (0,1), (0,2), (1,2)
@@ -579,7 +606,7 @@ __device__ __forceinline__ void q1_elastic_elements(const ElasticJob<T>& J, long
   }
   const int n = lane >> 3, m = lane & 7;
   const long long stride = (long long)J.gnx * GS::B2;  // GRID
-  for (int half = 0; half < 2; ++half) {
+  for (int half = 0; kHalf * half < turns; ++half) {
     __syncthreads();
     if ((i8 >> 2) == half) {
 #pragma unroll
@@ -588,7 +615,7 @@ __device__ __forceinline__ void q1_elastic_elements(const ElasticJob<T>& J, long
         for (int k = 0; k < 3; ++k) sB[wv][i8 & 3][q][a][k] = B[a][k];
     }
     __syncthreads();
-    for (int h = 0; h < kHalf; ++h) {
+    for (int h = 0; h < kHalf && kHalf * half + h < turns; ++h) {
       const int it = kHalf * half + h;
       const bool on = __builtin_amdgcn_readlane((int)active, 8 * it) != 0;
       T P[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -653,15 +680,15 @@ __device__ __forceinline__ void q1_elastic_elements(const ElasticJob<T>& J, long
 // entries stored straight from registers in runs of four values.
 template <typename T, bool GRID>
 __global__ __launch_bounds__(256) void q1_elastic_kernel(ElasticJob<T> J, const int32_t* __restrict__ order,
-                                                         int elem_begin, int elem_count,
+                                                         int elem_begin, int elem_count, int turns,
                                                          const double* __restrict__ dN, const double* __restrict__ w,
                                                          bool atomic) {
   const int blk = GRID ? GridStripe<8, 3>::block(J.gnx) : (int)blockIdx.x;
-  const int idx = blk * kQ1Elems + q1_elastic_slot();
-  const bool active = idx < elem_count;
+  const int slot = q1_elastic_slot(), idx = blk * 4 * turns + slot;
+  const bool active = slot < 4 * turns && idx < elem_count;
   long long e = 0;
   if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
-  q1_elastic_elements<T, GRID>(J, e, active, dN, w, atomic);
+  q1_elastic_elements<T, GRID>(J, e, active, turns, dN, w, atomic);
 }
 
 // ------------------------------------------- many meshes in one launch
@@ -705,14 +732,14 @@ __device__ __forceinline__ const BatchSeg& batch_seg(const BatchSeg* __restrict_
   return segs[lo];
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void scalar_batch_kernel(const BatchJob* __restrict__ jobs,
+template <typename T, int E, int G>
+__global__ __launch_bounds__(8 * E * G) void scalar_batch_kernel(const BatchJob* __restrict__ jobs,
                                                            const BatchSeg* __restrict__ segs, int nseg, int total,
                                                            const double* __restrict__ dN,
                                                            const double* __restrict__ N,
                                                            const double* __restrict__ w) {
-  for (int base = blockIdx.x * kQ1Elems; base < total; base += gridDim.x * kQ1Elems) {
-    const int idx = base + (threadIdx.x >> 3);
+  for (int base = blockIdx.x * E; base < total; base += gridDim.x * E) {
+    const int idx = base + threadIdx.x / (8 * G);
     const bool active = idx < total;
     ScalarJob<T> J{};
     long long e = 0;
@@ -722,18 +749,19 @@ __global__ __launch_bounds__(256) void scalar_batch_kernel(const BatchJob* __res
       J = ScalarJob<T>{B.coords, B.enodes, B.edofs, B.coef, B.source, B.pos, (T*)B.vals, B.svec, nullptr, 0, 0};
       e = B.order[sg.begin + idx - sg.prefix];
     }
-    q1_scalar_elements<T, false>(J, e, active, dN, N, w, false);
+    q1_scalar_elements<T, false, E, G>(J, e, active, dN, N, w, false);
   }
 }
 
 template <typename T>
 __global__ __launch_bounds__(256) void elastic_batch_kernel(const BatchJob* __restrict__ jobs,
                                                             const BatchSeg* __restrict__ segs, int nseg, int total,
+                                                            int turns,
                                                             const double* __restrict__ dN,
                                                             const double* __restrict__ w) {
-  for (int base = blockIdx.x * kQ1Elems; base < total; base += gridDim.x * kQ1Elems) {
-    const int idx = base + q1_elastic_slot();
-    const bool active = idx < total;
+  for (int base = blockIdx.x * 4 * turns; base < total; base += gridDim.x * 4 * turns) {
+    const int slot = q1_elastic_slot(), idx = base + slot;
+    const bool active = slot < 4 * turns && idx < total;
     ElasticJob<T> J{};
     long long e = 0;
     if (active) {
@@ -742,8 +770,40 @@ __global__ __launch_bounds__(256) void elastic_batch_kernel(const BatchJob* __re
       J = ElasticJob<T>{B.coords, B.enodes, B.coef, B.pos, (T*)B.vals, 0, 0};
       e = B.order[sg.begin + idx - sg.prefix];
     }
-    q1_elastic_elements<T, false>(J, e, active, dN, w, false);
+    q1_elastic_elements<T, false>(J, e, active, turns, dN, w, false);
   }
+}
+
+// Trilinear scalar elements per block (E) and groups of eight lanes per element (G) from
+// the elements of a launch.  Few elements: a wavefront each, its eight groups taking a row
+// of the matrix; such launches are as long as one wavefront, and eight launches make a
+// coloured assembly (16^3 elements, 512 to a launch: 45 us, 65 with eight elements per
+// wavefront, 52 with an element per wavefront and sums in LDS; 24^3, 1,728 to a launch: 60,
+// 68, 62; 32^3: 88, 78, 82).  Then eight elements per wavefront, a wavefront per block;
+// from 200,000 elements blocks of four (100^3 atomic: 995 us FP64, 773 FP32 one by one,
+// 990 and 752 with four; 61 x 47 x 53 structured 74 and 76).
+template <typename F>
+static void q1_scalar_launch(long long count, F&& f) {
+  using std::integral_constant;
+  if (count < 2048) f(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+  else if (count < 200000) f(integral_constant<int, 8>{}, integral_constant<int, 1>{});
+  else f(integral_constant<int, 32>{}, integral_constant<int, 1>{});
+}
+
+// Elements that a wavefront of a trilinear elasticity launch takes, one after the other: as
+// few as leave the chip full.  FP64, us with 1 / 2 / 4 / 8: staged 8^3 elements 20 / 21 / 23 /
+// 28, 16^3 37 / 31 / 31 / 36, 24^3 75 / 58 / 53 / 50; coloured, an eighth of the elements to
+// a launch, 16^3 67 / 86 / 123 / 199, 32^3 225 / 201 / 215 / 271, 61 x 47 x 53 1203 / 1055 /
+// 1030 / 1114 (FP32, which holds more wavefronts: 609 / 600 / 641 / 574; 45^3 375 / 389 /
+// 353 / 366).  Atomic adds bound the atomic form: 1224 / 1236 / 1215 / 1261 there, FP32
+// 951 / 954 / 957 / 962.
+enum class Form { kStage, kColour, kAtomic };
+template <typename T>
+static int elastic_turns(long long count, Form form) {
+  if (form == Form::kAtomic) return 1;
+  if (form == Form::kStage) return count < 1024 ? 1 : count < 4096 ? 2 : count < 8192 ? 4 : 8;
+  if (sizeof(T) == 4) return count < 4096 ? 1 : count < 8192 ? 2 : count < 16384 ? 4 : 8;
+  return count < 4096 ? 1 : count < 16384 ? 2 : 4;
 }
 
 template <int DIM, int NN, int NG, typename T>
@@ -756,9 +816,12 @@ static int launch_scalar(const mife_element_desc* d, int n_elem, const double* c
   const int tk = prof::begin(s);
   auto launch = [&](const int32_t* ord, int begin, int count, bool atomic) {
     if constexpr (DIM == 3 && NN == 8 && NG == 8)
-      q1_scalar_kernel<T, false><<<div_up(count, kQ1Elems), 256, 0, s>>>(
-          ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec, nullptr, 0, 0}, ord, begin, count, d->dN,
-          d->N, d->w, atomic);
+      q1_scalar_launch(count, [&](auto per, auto groups) {
+        constexpr int E = decltype(per)::value, G = decltype(groups)::value;
+        q1_scalar_kernel<T, false, E, G><<<div_up(count, E), 8 * E * G, 0, s>>>(
+            ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec, nullptr, 0, 0}, ord, begin, count,
+            d->dN, d->N, d->w, atomic);
+      });
     else if constexpr (kMfma)
       q2_assemble_mfma_kernel<T, false><<<div_up(count, kQ2Waves), 64 * kQ2Waves, 0, s>>>(
           coords, enodes, edofs, kappa, source, pos, ord, begin, count, d->dN, d->N, d->w, vals, svec, atomic, nullptr,
@@ -786,8 +849,9 @@ static int launch_elastic(const mife_element_desc* d, int n_elem, const double* 
                           int ncol, T* vals, hipStream_t s) {
   const int tk = prof::begin(s);
   auto launch = [&](const int32_t* ord, int begin, int count, bool atomic) {
-    q1_elastic_kernel<T, false><<<div_up(count, kQ1Elems), 256, 0, s>>>(
-        ElasticJob<T>{coords, enodes, material, pos, vals, 0, 0}, ord, begin, count, d->dN, d->w, atomic);
+    const int turns = elastic_turns<T>(count, atomic ? Form::kAtomic : Form::kColour);
+    q1_elastic_kernel<T, false><<<div_up(count, 4 * turns), 256, 0, s>>>(
+        ElasticJob<T>{coords, enodes, material, pos, vals, 0, 0}, ord, begin, count, turns, d->dN, d->w, atomic);
   };
   if (!order) {
     launch(nullptr, 0, n_elem, true);
@@ -994,20 +1058,24 @@ static int launch_grid(const mife_element_desc* d, const int* ne, const double* 
   const int tk = prof::begin(s);
   // multiples of the XCD count
   [[maybe_unused]] const int grid_e = div_up(div_up(E, kQ2Waves), 8) * 8;
-  [[maybe_unused]] const int grid_q1 = div_up(div_up(E, kQ1Elems), 8) * 8;
   if constexpr (NC == 1) {
     if constexpr (NN == 27) {
       q2_assemble_mfma_kernel<T, true><<<grid_e, 64 * kQ2Waves, 0, s>>>(coords, enodes, nullptr, coef, source, nullptr,
                                                                         nullptr, 0, (int)E, d->dN, d->N, d->w, kst,
                                                                         nullptr, false, sst, ne[0], ne[1]);
     } else {
-      q1_scalar_kernel<T, true><<<grid_q1, 256, 0, s>>>(
-          ScalarJob<T>{coords, enodes, nullptr, coef, source, nullptr, kst, nullptr, sst, ne[0], ne[1]}, nullptr, 0,
-          (int)E, d->dN, d->N, d->w, false);
+      q1_scalar_launch(E, [&](auto per, auto groups) {
+        constexpr int PE = decltype(per)::value, G = decltype(groups)::value;
+        q1_scalar_kernel<T, true, PE, G><<<div_up(div_up(E, PE), 8) * 8, 8 * PE * G, 0, s>>>(
+            ScalarJob<T>{coords, enodes, nullptr, coef, source, nullptr, kst, nullptr, sst, ne[0], ne[1]}, nullptr, 0,
+            (int)E, d->dN, d->N, d->w, false);
+      });
     }
   } else {
-    q1_elastic_kernel<T, true><<<grid_q1, 256, 0, s>>>(ElasticJob<T>{coords, enodes, coef, nullptr, kst, ne[0], ne[1]},
-                                                       nullptr, 0, (int)E, d->dN, d->w, false);
+    const int turns = elastic_turns<T>(E, Form::kStage);
+    q1_elastic_kernel<T, true><<<div_up(div_up(E, 4 * turns), 8) * 8, 256, 0, s>>>(
+        ElasticJob<T>{coords, enodes, coef, nullptr, kst, ne[0], ne[1]}, nullptr, 0, (int)E, turns, d->dN, d->w,
+        false);
   }
   constexpr int R = P * (64 / (P * P + 2 * P));
   const int runs = div_up(P * ne[0] + 1, R);
@@ -1232,21 +1300,26 @@ extern "C" int mife_assemble_batch(const mife_element_desc* scalar_desc, const m
   const BatchSeg* ds = (const BatchSeg*)((char*)work + align256(sizeof(BatchJob) * n_jobs));
   const int tk = prof::begin(s);
   for (const Launch& L : launches) {
-    const int grid = std::max(1, std::min(div_up(L.total, kQ1Elems), kBatchGrid));
+    auto grid = [&](int per) { return std::max(1, std::min(div_up(L.total, per), kBatchGrid)); };
     if (L.kind == MIFE_JOB_SCALAR) {
-      if (prec == MIFE_F64)
-        scalar_batch_kernel<double><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
-                                                                   scalar_desc->dN, scalar_desc->N, scalar_desc->w);
-      else
-        scalar_batch_kernel<float><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
-                                                                  scalar_desc->dN, scalar_desc->N, scalar_desc->w);
+      q1_scalar_launch(L.total, [&](auto per, auto groups) {
+        constexpr int E = decltype(per)::value, G = decltype(groups)::value;
+        if (prec == MIFE_F64)
+          scalar_batch_kernel<double, E, G><<<grid(E), 8 * E * G, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, scalar_desc->dN,
+                                                                   scalar_desc->N, scalar_desc->w);
+        else
+          scalar_batch_kernel<float, E, G><<<grid(E), 8 * E * G, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, scalar_desc->dN,
+                                                                  scalar_desc->N, scalar_desc->w);
+      });
     } else {
-      if (prec == MIFE_F64)
-        elastic_batch_kernel<double><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
-                                                                    elastic_desc->dN, elastic_desc->w);
-      else
-        elastic_batch_kernel<float><<<grid, 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
-                                                                   elastic_desc->dN, elastic_desc->w);
+      auto elastic = [&](auto zero) {
+        using T = decltype(zero);
+        const int turns = elastic_turns<T>(L.total, Form::kColour);
+        elastic_batch_kernel<T><<<grid(4 * turns), 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, turns,
+                                                                elastic_desc->dN, elastic_desc->w);
+      };
+      if (prec == MIFE_F64) elastic(0.0);
+      else elastic(0.0f);
     }
   }
   prof::end(tk, s, prof::kAssembleBatch);
