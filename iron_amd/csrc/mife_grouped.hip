@@ -55,9 +55,9 @@ constexpr int kL = 8;                  // CSR: lanes per row
 constexpr int kRowsPerBlock = 256 / kL;
 constexpr int kCsrRows = 4 * kRowsPerBlock;
 constexpr int kSlicesPerBlock = 4;     // SELL: one slice per wavefront
-constexpr int kSell3Waves = 4;         // SELL3: one slice per block, its blocks dealt over the wavefronts
+constexpr int kSell3Waves = 4;         // SELL3: wavefronts that share a slice (or take one each, sell3_slices)
 constexpr int kSell3Rows = 3 * kSlice;
-constexpr int kUpdateBlocks = 4;       // blocks whose rows one block of the update takes
+constexpr int kUpdateBlocks = 4;       // blocks of one unit (SELL3: a slice) whose rows one block of the update takes
 
 struct SegState {
   double rz, beta, rr, bb, tol2, rr_true;
@@ -90,7 +90,7 @@ struct Block {
   int32_t part;  // index of this block's partial slot
   int32_t p0, p1;  // the segment's partial slots
   int32_t keep;    // SELL: read the matrix with plain loads (the Infinity Cache keeps it)
-  int32_t pad;
+  int32_t upd;     // blocks whose rows one block of the update takes
 };
 
 struct View {
@@ -141,6 +141,30 @@ __device__ __forceinline__ T slice_dot(const View& V, const mife_segment& S, boo
   return sell_row<T>(sp, V.col + S.nz_off, val, xs, s, lane);
 }
 
+// block_walk of a block whose wavefronts take a SELL3 slice each (Block::upd == 1): the hook
+// first, so that no register holds its operands during the product.
+template <typename T, typename P, typename F, typename H>
+__device__ __forceinline__ void wave_slices_walk(const View& V, const Block& B, const mife_segment& S,
+                                                 const T* __restrict__ vpool, const T* __restrict__ x, P&& pre, F&& f,
+                                                 H& hook) {
+  hook_now(hook);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (wave >= B.rows) return;
+  const int s = B.row0 + wave;
+  const int32_t* sp = V.rp + S.rp_off;
+  const int base = sp[s], len = (sp[s + 1] - base) / kSlice;
+  T ax[3];
+  const uint16_t* c16 = V.col16 + S.nz_off + base + lane;
+  const T* v = vpool + S.nz_off + (size_t)9 * base + lane;
+  const T* xs = x + S.row_off + 3 * (size_t)V.cbase[S.cb_off + s];
+  if (B.keep) sell3_sum<T, T, false>(c16, v, xs, len, 0, 1, ax);
+  else sell3_sum<T, T, true>(c16, v, xs, len, 0, 1, ax);
+  const int row = s * kSell3Rows + 3 * lane;
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    if (row + c < S.n) f(row + c, ax[c], pre(row + c));
+}
+
 // Calls f(row, (A x)_row, pre(row)) for every row of block B (by one lane per row).
 // On the SELL storages pre's loads and the hook's are in flight during the product;
 // hook.stage() and hook.finish() run once per block, a barrier apart, before any f.
@@ -150,6 +174,10 @@ __device__ __forceinline__ void block_walk(const View& V, const Block& B, const 
                                            H& hook) {
   using PV = decltype(pre(0));
   PV pv = {};
+  if (B.upd == 1) {
+    wave_slices_walk<T>(V, B, S, vpool, x, pre, f, hook);
+    return;
+  }
   if (S.format == MIFE_FMT_SELL3 && B.rows > 0) {
     // node rows: lane k of the slice gives rows 3 (64 s + k) + c; block columns in
     // the 16-bit column pool at the segment's value offset.  The wavefronts' shares
@@ -220,14 +248,14 @@ __device__ __forceinline__ void block_row_range(const Block& B, const mife_segme
 
 // Partials of a segment's updates, and the rows of one of them.
 __device__ __forceinline__ int update_blocks(const Block& B) {
-  return (B.p1 - B.p0 + kUpdateBlocks - 1) / kUpdateBlocks;
+  return (B.p1 - B.p0 + B.upd - 1) / B.upd;
 }
 __device__ __forceinline__ void update_row_range(const Block& B, const mife_segment& S, int& r0, int& r1) {
   const bool csr = S.format == MIFE_FMT_CSR;
-  const int per = csr ? kCsrRows : S.format == MIFE_FMT_SELL3 ? 1 : kSlicesPerBlock;
+  const int units = kUpdateBlocks * (csr ? kCsrRows : S.format == MIFE_FMT_SELL3 ? 1 : kSlicesPerBlock);
   Block all = B;
-  all.row0 = (B.part - B.p0) * kUpdateBlocks * per;
-  all.rows = min(kUpdateBlocks * per, (csr ? S.n : S.n_slices) - all.row0);
+  all.row0 = (B.part - B.p0) * units;
+  all.rows = min(units, (csr ? S.n : S.n_slices) - all.row0);
   block_row_range(all, S, r0, r1);
 }
 
@@ -740,6 +768,16 @@ size_t mife_grouped_work_bytes(int max_segments, int max_blocks) {
   return b;
 }
 
+// Slices that a block of a SELL3 product takes: one, its wavefronts sharing it, or four, one
+// each.  Sharing gives a small segment blocks enough for the chip.  A large one has them
+// anyway, and then long runs per wavefront, a quarter of the partials and a hook before the
+// product cost less.  Shared / one each, ms for one elasticity request to 1e-8, FP64: 810
+// slices 49.7 / 55.2, 1,451 86.4 / 88.8, 1,871 133.6 / 127.8, 3,600 305.6 / 289.9 (product 96
+// -> 91 us, update 13 -> 10); FP32 with FP64 replacements: 810 slices 88.1 / 88.5, 1,099 123
+// / 113, 1,871 219 / 215, 3,600 545 / 446.  By the segment's own size alone, so that its
+// sums do not depend on what it shares a launch with.
+static int sell3_slices(int n_slices, int prec) { return n_slices < (prec == MIFE_F32 ? 1000 : 1700) ? 1 : 4; }
+
 int mife_grouped_blocks(int n_rows) { return std::max(1, div_up(n_rows, kCsrRows)); }
 
 int mife_grouped_setup(const mife_segment* segs_host, int n_seg, int max_segments, int max_blocks,
@@ -766,7 +804,7 @@ int mife_grouped_setup(const mife_segment* segs_host, int n_seg, int max_segment
     H.seg_parts[k] = nb;
     H.seg_ids[k] = S.slot;
     const bool sell = S.format != MIFE_FMT_CSR;
-    const int per = S.format == MIFE_FMT_SELL3 ? 1 : sell ? kSlicesPerBlock : kCsrRows;
+    const int per = S.format == MIFE_FMT_SELL3 ? sell3_slices(S.n_slices, S.prec) : sell ? kSlicesPerBlock : kCsrRows;
     const int units = sell ? S.n_slices : S.n;
     // as many matrices as the Infinity Cache holds stay there between the products; their
     // sizes are not in the table, so trilinear rows are assumed (a wrong guess costs
@@ -778,7 +816,8 @@ int mife_grouped_setup(const mife_segment* segs_host, int n_seg, int max_segment
     int r0 = 0;
     do {
       MIFE_REQUIRE(nb < max_blocks, MIFE_ERR_ARG, "block table full (%d blocks)", max_blocks);
-      H.blocks[nb] = Block{S.slot, r0, std::max(0, std::min(per, units - r0)), nb, p0, p1, keep, 0};
+      H.blocks[nb] = Block{S.slot, r0, std::max(0, std::min(per, units - r0)), nb, p0, p1, keep,
+                            S.format == MIFE_FMT_SELL3 ? kUpdateBlocks / per : kUpdateBlocks};
       ++nb;
       r0 += per;
     } while (r0 < units);

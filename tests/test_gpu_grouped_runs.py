@@ -52,3 +52,23 @@ def test_fp64_segment_next_to_mixed_ones():
     assert len(kept) == 1
     for k in kept:
         assert split[k].iterations == fp64[k].iterations and np.array_equal(split[k].u, fp64[k].u)
+
+
+@pytest.mark.parametrize("ne", [(67, 39, 39), (68, 39, 39), (40, 39, 38), (40, 39, 39)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_elasticity_with_a_slice_per_wavefront(ne, precision):
+    """Slice counts below and at those from which a block's wavefronts take a SELL3 slice
+    each: 1,700 (FP64) and 1,000 (FP32), nodes nx (ny + 1)(nz + 1) in slices of 64."""
+    from iron_amd import serving
+    print(f"case grouped SELL3 {ne} {precision}", flush=True)
+
+    def req():
+        return serving.Request(0, "elasticity", ne, 17, rtol=1e-9)
+
+    ref = _serve([req()], 2e9, precision=precision, chunk=16)[0]
+    one = serving.solve_one_fp64(req(), {})
+    # two solves to 1e-9 of systems with condition numbers up to 1e5
+    assert np.abs(ref.u - one.u).max() <= 1e-4 * np.abs(one.u).max()
+    if precision == "fp64":
+        other = _serve([req()], 2e9, precision=precision, chunk=7)[0]
+        assert other.iterations == ref.iterations and np.array_equal(other.u, ref.u)
