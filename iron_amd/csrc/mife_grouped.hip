@@ -138,7 +138,8 @@ __device__ __forceinline__ T slice_dot(const View& V, const mife_segment& S, boo
     return keep ? sell16_row<T, T, false>(sp, c16, cb, val, xs, s, lane)
                 : sell16_row<T, T, true>(sp, c16, cb, val, xs, s, lane);
   }
-  return sell_row<T>(sp, V.col + S.nz_off, val, xs, s, lane);
+  const int32_t* c32 = V.col + S.nz_off;
+  return keep ? sell_row<T, T, false>(sp, c32, val, xs, s, lane) : sell_row<T, T, true>(sp, c32, val, xs, s, lane);
 }
 
 // block_walk of a block whose wavefronts take a SELL3 slice each (Block::upd == 1): the hook
@@ -224,11 +225,13 @@ __device__ __forceinline__ void block_walk(const View& V, const Block& B, const 
   }
 }
 
-// Calls f(row, (A x)_row) for every row of block B (by one lane per row).
+// Calls f(row, (A x)_row) for every row of a block (by one lane per row); for passes that
+// read a matrix once between products: nothing of it is kept.
 template <typename T, typename F>
-__device__ __forceinline__ void block_rows(const View& V, const Block& B, const mife_segment& S,
+__device__ __forceinline__ void block_rows(const View& V, Block B, const mife_segment& S,
                                            const T* __restrict__ vpool, const T* __restrict__ x, F&& f) {
   NoHook none;
+  B.keep = 0;
   block_walk<T>(V, B, S, vpool, x, [](int) { return 0; }, [&](int row, T ax, int) { f(row, ax); }, none);
 }
 
@@ -806,10 +809,14 @@ int mife_grouped_setup(const mife_segment* segs_host, int n_seg, int max_segment
     const bool sell = S.format != MIFE_FMT_CSR;
     const int per = S.format == MIFE_FMT_SELL3 ? sell3_slices(S.n_slices, S.prec) : sell ? kSlicesPerBlock : kCsrRows;
     const int units = sell ? S.n_slices : S.n;
-    // as many matrices as the Infinity Cache holds stay there between the products; their
-    // sizes are not in the table, so trilinear rows are assumed (a wrong guess costs
-    // cache hits, nothing else)
-    const double bytes = 27.0 * S.n * (S.format == MIFE_FMT_SELL3 ? 24.7 : 10.0);
+    // as many matrices as the Infinity Cache holds stay there between the products.  A
+    // product reads a value of the segment's precision and its share of a column per
+    // entry; how many entries a row has is not in the table, so trilinear rows are assumed
+    // (a wrong guess costs cache hits, nothing else)
+    const bool nodes = S.format == MIFE_FMT_SELL3;
+    const double value = S.prec == MIFE_F32 ? 4.0 : 8.0;
+    const double column = nodes ? 2.0 / 9.0 : S.cb_off >= 0 && S.format == MIFE_FMT_SELL ? 2.0 : 4.0;
+    const double bytes = (nodes ? 81.0 : 27.0) * S.n * (value + column);
     const int keep = kept + bytes <= kKeepMost ? 1 : 0;
     if (keep) kept += bytes;
     const int p0 = nb, p1 = nb + std::max(1, div_up(units, per));

@@ -13,10 +13,10 @@ SHIM = ROOT / "tests" / "host_shim"
 CLANG = next((c for c in ("/opt/rocm/llvm/bin/clang++", shutil.which("clang++")) if c and Path(c).exists()), None)
 
 
-def device_part(name):
+def device_part(name, until="host side", close="}\n"):
     """A .hip file up to its host side: kernels and what they use, namespace closed."""
     text = (CSRC / name).read_text()
-    return text[:text.index("host side")].rsplit("\n", 1)[0] + "\n}\n"
+    return text[:text.index(until)].rsplit("\n", 1)[0] + "\n" + close
 
 
 def definition(name, what):

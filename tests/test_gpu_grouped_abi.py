@@ -149,3 +149,41 @@ def test_grouped_abi_all_storages_and_precisions():
             out[perm.cpu().numpy()] = xk
             xk = out
         assert np.abs(xk - xref).max() <= 1e-8 * max(1.0, np.abs(xref).max()), k
+
+
+def test_grouped_table_keeps_what_the_cache_holds():
+    """The table marks segments as kept, in its order, while the bytes that their products
+    read (27 entries per row, 81 of node blocks; values of the segment's precision and
+    16-bit, int32 or per-block columns) fit 210 MB; later ones may still fit."""
+    from iron_amd import _lib
+    from iron_amd._lib import Segment
+    print("case grouped table: kept segments", flush=True)
+    MB = 1e6
+    per_row = {("csr", "f64"): 27 * 12, ("sell32", "f64"): 27 * 12, ("sell32", "f32"): 27 * 8, ("sell16", "f64"): 27 * 10,
+               ("sell16", "f32"): 27 * 6, ("sell3", "f64"): 81 * (8 + 2 / 9), ("sell3", "f32"): 81 * (4 + 2 / 9)}
+    groups = [[("sell16", "f64", 100), ("sell16", "f64", 109), ("sell16", "f64", 2), ("sell16", "f64", 0.5)],
+              [("sell16", "f32", 209), ("sell16", "f64", 2)], [("sell32", "f64", 120), ("sell32", "f32", 89), ("sell3", "f64", 2)],
+              [("sell3", "f32", 209), ("sell3", "f64", 0.5)], [("sell3", "f64", 211), ("sell3", "f64", 209)]]
+    fmt = {"csr": _lib.MIFE_FMT_CSR, "sell32": _lib.MIFE_FMT_SELL, "sell16": _lib.MIFE_FMT_SELL, "sell3": _lib.MIFE_FMT_SELL3}
+    L = _lib.lib()
+    for group in groups:
+        segs, want, kept, blocks = [], [], 0.0, 0
+        for slot, (kind, prec, mb) in enumerate(group):
+            n = 192 * int(mb * MB / per_row[kind, prec] / 192)
+            ns = 0 if kind == "csr" else -(-n // (192 if kind == "sell3" else 64))
+            segs.append(Segment(n, 1, slot, fmt[kind], 0, 0, 0, 1e-8, ns, 0 if prec == "f64" else 1,
+                                0 if kind in ("sell16", "sell3") else -1))
+            size = n * per_row[kind, prec]
+            want.append(int(kept + size <= 210 * MB))
+            kept += size * want[-1]
+            blocks += L.mife_grouped_blocks(n)
+        k = len(segs)
+        table = np.zeros(L.mife_grouped_work_bytes(k, blocks), dtype=np.uint8)
+        work = torch.zeros(table.size, dtype=torch.uint8, device="cuda")
+        nb = C.c_int(0)
+        _lib.call("mife_grouped_setup", (Segment * k)(*segs), k, k, blocks, C.byref(nb), table.ctypes.data, _lib.ptr(work),
+                  None)
+        off = -(-C.sizeof(Segment) * k // 256) * 256
+        b = table[off: off + 32 * nb.value].view(np.int32).reshape(-1, 8)
+        for slot in range(k):
+            assert set(b[b[:, 0] == slot, 6]) == {want[slot]}, (group, slot)

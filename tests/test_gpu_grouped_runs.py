@@ -72,3 +72,21 @@ def test_elasticity_with_a_slice_per_wavefront(ne, precision):
     if precision == "fp64":
         other = _serve([req()], 2e9, precision=precision, chunk=7)[0]
         assert other.iterations == ref.iterations and np.array_equal(other.u, ref.u)
+
+
+def test_streamed_segments_beside_kept_ones():
+    """A group beyond what the cache keeps (the first two diffusion requests fit it, the
+    third and the elasticity one do not): every solution is that of the request served
+    alone, where it is kept, bit for bit."""
+    from iron_amd import serving
+    print("case grouped runs: kept and streamed segments", flush=True)
+
+    def reqs():
+        return [serving.Request(k, kind, ne, 40 + k, rtol=1e-8) for k, (kind, ne) in enumerate([
+            ("diffusion", (65, 74, 73)), ("diffusion", (66, 60, 73)), ("diffusion", (75, 74, 73)),
+            ("elasticity", (40, 24, 22))])]
+
+    both = _serve(reqs(), 8e9, precision="fp64", chunk=16)
+    for r in reqs():
+        alone = _serve([r], 8e9, precision="fp64", chunk=16)[r.rid]
+        assert alone.iterations == both[r.rid].iterations and np.array_equal(alone.u, both[r.rid].u), r.rid
