@@ -1177,7 +1177,7 @@ static bool g_graphs_on = true;
 static int g_gmres_refine = 0;
 
 struct GraphKey {
-  int dev, tsize, n, fmt, n_slices, span, split, L;
+  int dev, tsize, n, fmt, n_slices, span, split, L, keep64, keep32;
   const void* ptrs[13];
   bool operator==(const GraphKey& o) const { return std::memcmp(this, &o, sizeof(GraphKey)) == 0; }
 };
@@ -1207,6 +1207,8 @@ static int cg_chunk_graph(const Mat& M, const T* vals, T* x, T* r, T* z, T* p, T
   key.span = M.a.span;
   key.split = M.a.split;
   key.L = M.L;
+  key.keep64 = M.a.keep64;
+  key.keep32 = M.a.keep32;
   const void* ps[13] = {M.a.ptr, M.a.col, M.a.cbase, M.a.order, vals, x, r, z, p, q, dinv, st, nullptr};
   std::memcpy(key.ptrs, ps, sizeof(ps));
   std::lock_guard<std::mutex> lock(g_graph_mu);

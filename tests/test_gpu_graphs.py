@@ -68,3 +68,19 @@ def test_graph_replays_equal_eager_launches(mixed):
         finally:
             _lib.graphs_enable(True)
         assert np.array_equal(x_e, ref)
+
+
+def test_graphs_are_kept_apart_by_cache_policy():
+    """Two descriptors of one matrix that state different sizes replay different graphs: the
+    captured kernels hold the part of the matrix that is read with plain loads."""
+    from iron_amd import _lib
+    print("case CG graph key: cache policy", flush=True)
+    fem, red, S, s64, s32, bvec = _system()
+    ws = fem.KrylovWorkspace(red.n_free, "cuda")
+    stored, before, x = S.desc.nnz, _lib.lib().mife_graphs_cached(), []
+    for nnz in (25_000_000, 40_000_000):  # 13 and 8 sixteenths kept; the same lanes per row
+        S.desc.nnz = nnz
+        x.append(_solve(fem, red, S, s64, s32, bvec, ws, False)[0])
+    S.desc.nnz = stored
+    assert np.array_equal(x[0], x[1])
+    assert _lib.lib().mife_graphs_cached() == min(before + 2, 16)  # 16: the graphs kept in all
