@@ -74,13 +74,22 @@ __device__ __forceinline__ void add_values(T* const (&at)[N], const T (&v)[N], b
     if (at[k]) *at[k] = old[k] + v[k];
 }
 
-// As above for entries p of one CSR (p < 0: none).
+// As above for entries p of one CSR (p < 0: none), an index instead of an address each (with
+// addresses the triquadratic scatter of 1,000 elements took 113 us instead of 108).
 template <typename T, int N>
 __device__ __forceinline__ void add_values(T* __restrict__ vals, const int (&p)[N], const T (&v)[N], bool atomic) {
-  T* at[N];
+  if (atomic) {
 #pragma unroll
-  for (int k = 0; k < N; ++k) at[k] = p[k] >= 0 ? vals + p[k] : nullptr;
-  add_values(at, v, atomic);
+    for (int k = 0; k < N; ++k)
+      if (p[k] >= 0) atomicAdd(&vals[p[k]], v[k]);
+    return;
+  }
+  T old[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) old[k] = p[k] >= 0 ? vals[p[k]] : (T)0;
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    if (p[k] >= 0) vals[p[k]] = old[k] + v[k];
 }
 
 // Stage layout of a structured (grid) assembly.  With row m = (c, a), column
@@ -793,17 +802,17 @@ static void q1_scalar_launch(long long count, F&& f) {
 // Elements that a wavefront of a trilinear elasticity launch takes, one after the other: as
 // few as leave the chip full.  FP64, us with 1 / 2 / 4 / 8: staged 8^3 elements 20 / 21 / 23 /
 // 28, 16^3 37 / 31 / 31 / 36, 24^3 75 / 58 / 53 / 50; coloured, an eighth of the elements to
-// a launch, 16^3 67 / 86 / 123 / 199, 32^3 225 / 201 / 215 / 271, 61 x 47 x 53 1203 / 1055 /
-// 1030 / 1114 (FP32, which holds more wavefronts: 609 / 600 / 641 / 574; 45^3 375 / 389 /
-// 353 / 366).  Atomic adds bound the atomic form: 1224 / 1236 / 1215 / 1261 there, FP32
-// 951 / 954 / 957 / 962.
+// a launch, 16^3 67 / 86 / 123 / 199, 32^3 225 / 201 / 215 / 271, 45^3 630 / 553 / 570 / 545
+// (at 8 all its blocks are resident), 61 x 47 x 53 1203 / 1055 / 1030 / 1114.  FP32 holds more
+// wavefronts: 45^3 375 / 389 / 353 / 366, 61 x 47 x 53 609 / 600 / 641 / 574.  Atomic adds
+// bound the atomic form: 1224 / 1236 / 1215 / 1261 there, FP32 951 / 954 / 957 / 962.
 enum class Form { kStage, kColour, kAtomic };
 template <typename T>
 static int elastic_turns(long long count, Form form) {
-  if (form == Form::kAtomic) return 1;
+  if (form == Form::kAtomic) return sizeof(T) == 4 || count < 8192 ? 1 : 4;
   if (form == Form::kStage) return count < 1024 ? 1 : count < 4096 ? 2 : count < 8192 ? 4 : 8;
   if (sizeof(T) == 4) return count < 4096 ? 1 : count < 8192 ? 2 : count < 16384 ? 4 : 8;
-  return count < 4096 ? 1 : count < 16384 ? 2 : 4;
+  return count < 4096 ? 1 : count < 8192 ? 2 : count < 16384 ? 8 : 4;
 }
 
 template <int DIM, int NN, int NG, typename T>
