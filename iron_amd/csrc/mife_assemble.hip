@@ -22,28 +22,38 @@ struct Mat3 {
   double a[3][3];
 };
 
-// 2x2 / 3x3 inverse by cofactors (maths.F90 InvertFullDP ordering of terms).
+// 2x2 / 3x3 inverse by cofactors (maths.F90 InvertFullDP ordering of terms), every
+// multiply-add written out: the bits do not depend on what the compiler fuses around it.
 template <int DIM>
 __device__ __forceinline__ double invert(const double (&A)[3][3], double (&B)[3][3]) {
+#pragma clang fp contract(off)
+  // a b - c d
+  auto minor = [](double a, double b, double c, double d) {
+#pragma clang fp contract(off)
+    return fma(a, b, -(c * d));
+  };
   if constexpr (DIM == 2) {
-    const double det = A[0][0] * A[1][1] - A[1][0] * A[0][1];
+    const double det = minor(A[0][0], A[1][1], A[1][0], A[0][1]);
     B[0][0] = A[1][1] / det;
     B[0][1] = -A[0][1] / det;
     B[1][0] = -A[1][0] / det;
     B[1][1] = A[0][0] / det;
     return det;
   } else {
-    const double det = A[0][0] * A[1][1] * A[2][2] + A[0][1] * A[1][2] * A[2][0] + A[0][2] * A[1][0] * A[2][1] -
-                       A[0][0] * A[2][1] * A[1][2] - A[1][0] * A[0][1] * A[2][2] - A[2][0] * A[1][1] * A[0][2];
-    B[0][0] = (A[1][1] * A[2][2] - A[2][1] * A[1][2]) / det;
-    B[1][0] = (A[1][2] * A[2][0] - A[2][2] * A[1][0]) / det;
-    B[2][0] = (A[1][0] * A[2][1] - A[2][0] * A[1][1]) / det;
-    B[0][1] = (A[2][1] * A[0][2] - A[0][1] * A[2][2]) / det;
-    B[1][1] = (A[2][2] * A[0][0] - A[0][2] * A[2][0]) / det;
-    B[2][1] = (A[2][0] * A[0][1] - A[0][0] * A[2][1]) / det;
-    B[0][2] = (A[0][1] * A[1][2] - A[1][1] * A[0][2]) / det;
-    B[1][2] = (A[0][2] * A[1][0] - A[1][2] * A[0][0]) / det;
-    B[2][2] = (A[0][0] * A[1][1] - A[1][0] * A[0][1]) / det;
+    double det = fma(A[0][0] * A[1][1], A[2][2], (A[0][1] * A[1][2]) * A[2][0]);
+    det = fma(A[0][2] * A[1][0], A[2][1], det);
+    det = fma(-(A[0][0] * A[2][1]), A[1][2], det);
+    det = fma(-(A[1][0] * A[0][1]), A[2][2], det);
+    det = fma(-(A[2][0] * A[1][1]), A[0][2], det);
+    B[0][0] = minor(A[1][1], A[2][2], A[2][1], A[1][2]) / det;
+    B[1][0] = minor(A[1][2], A[2][0], A[2][2], A[1][0]) / det;
+    B[2][0] = minor(A[1][0], A[2][1], A[2][0], A[1][1]) / det;
+    B[0][1] = minor(A[2][1], A[0][2], A[0][1], A[2][2]) / det;
+    B[1][1] = minor(A[2][2], A[0][0], A[0][2], A[2][0]) / det;
+    B[2][1] = minor(A[2][0], A[0][1], A[0][0], A[2][1]) / det;
+    B[0][2] = minor(A[0][1], A[1][2], A[1][1], A[0][2]) / det;
+    B[1][2] = minor(A[0][2], A[1][0], A[1][2], A[0][0]) / det;
+    B[2][2] = minor(A[0][0], A[1][1], A[1][0], A[0][1]) / det;
     return det;
   }
 }
