@@ -213,8 +213,13 @@ struct ScalarJob {
   const int32_t* pos;   // NULL: structured (the element matrices go to the stage at vals)
   T* vals;
   double* svec;
-  double* sstage;       // non-NULL: stage the element source vector at sstage[e][NN]
-  int gnx, gny;         // GRID: elements in x and y (GridStripe layout)
+};
+
+// Where a structured assembly's element source vectors go ([e][NN], or NULL), and its
+// elements in x and y (GridStripe layout).
+struct ScalarStage {
+  double* source = nullptr;
+  int gnx = 0, gny = 0;
 };
 
 // One element per wavefront (element e when `active`); every wavefront of the
@@ -279,8 +284,7 @@ __global__ __launch_bounds__(64 * WPB) void scalar_assemble_kernel(
   long long e = 0;
   if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
   scalar_element<DIM, NN, NG, T, WPB>(
-      ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec, nullptr, 0, 0}, e, active, dN, N, w,
-      atomic);
+      ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec}, e, active, dN, N, w, atomic);
 }
 
 // ------------------------------------------------ trilinear elements, eight per wavefront
@@ -330,7 +334,7 @@ __device__ __forceinline__ double q1_geometry(Q1Tables<E>& S, const double* __re
 // One scalar element per 8 G lanes (e and J are those lanes' own); every thread of the
 // block calls it.
 template <typename T, bool GRID, int E, int G>
-__device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, long long e, bool active,
+__device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, const ScalarStage& Q, long long e, bool active,
                                                    const double* __restrict__ dN, const double* __restrict__ N,
                                                    const double* __restrict__ w, bool atomic) {
 #pragma clang fp contract(off)
@@ -372,10 +376,10 @@ __device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, long l
 #pragma unroll
       for (int n = m; n < 8; ++n, ++t) entry(m, n, B[m], q == (t & 7));
   }
-  if (GRID && q == 0 && g == 0) sbase[el] = active ? GS::base(e, J.gnx, J.gny) : -1;
+  if (GRID && q == 0 && g == 0) sbase[el] = active ? GS::base(e, Q.gnx, Q.gny) : -1;
   __syncthreads();
   if constexpr (GRID) {
-    GS::template store<T, E>(sK, sbase, J.gnx, J.vals);
+    GS::template store<T, E>(sK, sbase, Q.gnx, J.vals);
   } else {
     // the wavefront's elements one by one, a lane per entry: the lanes of a store lie in
     // eight rows (a row per lane instead, in eight elements at once, touched 64 lines:
@@ -394,13 +398,13 @@ __device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, long l
     }
     add_values(at, v, atomic);
   }
-  if (active && g == 0 && J.source && (J.svec || J.sstage)) {
+  if (active && g == 0 && J.source && (J.svec || Q.source)) {
     double s = 0.0;
 #pragma unroll
     for (int p = 0; p < 8; ++p) s = fma(N[p * 8 + q], rw[el][p], s);
     s = s * J.source[e];
-    if (J.sstage)
-      J.sstage[e * 8 + q] = s;
+    if (Q.source)
+      Q.source[e * 8 + q] = s;
     else
       add_value(&J.svec[J.edofs[e * 8 + q]], s, atomic);
   }
@@ -409,16 +413,16 @@ __device__ __forceinline__ void q1_scalar_elements(const ScalarJob<T>& J, long l
 // Measured on 61 x 47 x 53 elements with moved nodes, FP64, structured: 187 us with
 // one element per wavefront, 55 us now (78 MB of element matrices stored).
 template <typename T, bool GRID, int E, int G>
-__global__ __launch_bounds__(8 * E * G) void q1_scalar_kernel(ScalarJob<T> J, const int32_t* __restrict__ order,
+__global__ __launch_bounds__(8 * E * G) void q1_scalar_kernel(ScalarJob<T> J, ScalarStage Q, const int32_t* __restrict__ order,
                                                         int elem_begin, int elem_count,
                                                         const double* __restrict__ dN, const double* __restrict__ N,
                                                         const double* __restrict__ w, bool atomic) {
-  const int blk = GRID ? GridStripe<8, 1>::block(J.gnx) : (int)blockIdx.x;
+  const int blk = GRID ? GridStripe<8, 1>::block(Q.gnx) : (int)blockIdx.x;
   const int idx = blk * E + (threadIdx.x / (8 * G));
   const bool active = idx < elem_count;
   long long e = 0;
   if (active) e = order ? order[elem_begin + idx] : (long long)elem_begin + idx;
-  q1_scalar_elements<T, GRID, E, G>(J, e, active, dN, N, w, atomic);
+  q1_scalar_elements<T, GRID, E, G>(J, Q, e, active, dN, N, w, atomic);
 }
 
 // ------------------------------------------------ triquadratic, on MFMA
@@ -765,10 +769,10 @@ __global__ __launch_bounds__(8 * E * G) void scalar_batch_kernel(const BatchJob*
     if (active) {
       const BatchSeg sg = batch_seg(segs, nseg, idx);
       const BatchJob B = jobs[sg.job];
-      J = ScalarJob<T>{B.coords, B.enodes, B.edofs, B.coef, B.source, B.pos, (T*)B.vals, B.svec, nullptr, 0, 0};
+      J = ScalarJob<T>{B.coords, B.enodes, B.edofs, B.coef, B.source, B.pos, (T*)B.vals, B.svec};
       e = B.order[sg.begin + idx - sg.prefix];
     }
-    q1_scalar_elements<T, false, E, G>(J, e, active, dN, N, w, false);
+    q1_scalar_elements<T, false, E, G>(J, ScalarStage{}, e, active, dN, N, w, false);
   }
 }
 
@@ -838,7 +842,7 @@ static int launch_scalar(const mife_element_desc* d, int n_elem, const double* c
       q1_scalar_launch(count, [&](auto per, auto groups) {
         constexpr int E = decltype(per)::value, G = decltype(groups)::value;
         q1_scalar_kernel<T, false, E, G><<<div_up(count, E), 8 * E * G, 0, s>>>(
-            ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec, nullptr, 0, 0}, ord, begin, count,
+            ScalarJob<T>{coords, enodes, edofs, kappa, source, pos, vals, svec}, ScalarStage{}, ord, begin, count,
             d->dN, d->N, d->w, atomic);
       });
     else if constexpr (kMfma)
@@ -1086,7 +1090,8 @@ static int launch_grid(const mife_element_desc* d, const int* ne, const double* 
       q1_scalar_launch(E, [&](auto per, auto groups) {
         constexpr int PE = decltype(per)::value, G = decltype(groups)::value;
         q1_scalar_kernel<T, true, PE, G><<<div_up(div_up(E, PE), 8) * 8, 8 * PE * G, 0, s>>>(
-            ScalarJob<T>{coords, enodes, nullptr, coef, source, nullptr, kst, nullptr, sst, ne[0], ne[1]}, nullptr, 0,
+            ScalarJob<T>{coords, enodes, nullptr, coef, source, nullptr, kst, nullptr},
+            ScalarStage{sst, ne[0], ne[1]}, nullptr, 0,
             (int)E, d->dN, d->N, d->w, false);
       });
     }

@@ -35,15 +35,15 @@ namespace mife {
 
 constexpr int kRedBlocks = kMaxSellGrid;  // partial slots per reduced value (largest row grid)
 constexpr int kMaxRestart = 256;
-constexpr int kFinThreads = 1024;  // one-block finishers: two partials per thread
+constexpr int kFinThreads = 1024;  // one-block finishers (up to kRedBlocks partials)
 // CG update blocks: 1024 threads, so that the blocks are few (one round) and each
 // sums K_A's partials once
 constexpr int kUpdateThreads = 1024;
 constexpr int kMaxIterChunk = 256;  // CG iterations launched between two host reads of the state
 
 struct CgScalars {
-  double rz, pq, alpha, beta, rr, bb, tol2, scale;
-  double rz_prev, maxrr, rr_seg, rr64;  // rr_seg: recurrence r.r when a segment ended
+  double rz, beta, rr, bb, tol2;
+  double rz_prev, rr_seg, rr64;  // rr_seg: recurrence r.r when a segment ended
   // Segmented (mixed-precision) solves: a segment pauses once r.r <= seg_rr, set at
   // each replacement to seg_drop x the new r.r (seg_drop = 0: no pausing).
   double seg_drop, seg_rr;
@@ -248,9 +248,7 @@ __global__ void fin_init_kernel(CgState* st, int nb, double tol2, int maxit) {
     c.rz = out[0];
     c.rr = out[1];
     c.bb = out[2];
-    c.maxrr = out[1];
     c.beta = 0.0;
-    c.alpha = 0.0;
     c.iters = 0;
     c.maxit = maxit;
     c.tol2 = tol2;
@@ -274,7 +272,6 @@ __device__ __forceinline__ void cg_advance(CgScalars& c, double rz, double rr) {
   c.rz = rz;
   c.rr = rr;
   c.iters += 1;
-  c.maxrr = fmax(c.maxrr, rr);
 }
 
 // Largest update grid: one block per CU, two partials per thread of a product block.
@@ -464,7 +461,6 @@ __global__ void fin_residual_kernel(CgState* st, int nb) {
     c.rr64 = out[0];
     c.rr = out[0];
     c.bb = out[1];
-    c.scale = sqrt(out[0]);
   }
 }
 
@@ -538,7 +534,6 @@ __global__ void fin_replace_kernel(CgState* st, const CgState* ro, int nb, int f
     c.beta = (first || out[1] > kRestartGrowth * c.rr) ? 0.0 : out[0] / c.rz_prev;
     c.rz = out[0];
     c.rr = out[1];
-    c.maxrr = out[1];
     c.bb = t.bb;
     c.pause = 0;
     // the next segment ends when the recurrence has fallen by seg_drop, or at a
@@ -1104,13 +1099,16 @@ static void launch_cg_init(const Mat& M, const T* vals, const T* b, const T* x, 
   prof::end(tk, s, prof::kCgInit);
 }
 
-// Grid of the update kernel (its partials are summed by every product block).
+// Whether the update kernel may read and write the vectors 16 bytes at a time.
 static bool update_vectorised(std::initializer_list<const void*> ps) {
   for (const void* p : ps)
     if (!aligned16(p)) return false;
   return true;
 }
 
+// Grid of the update kernel; every product block sums its partials, hence the limit.  Beyond
+// 256 blocks' worth of rows the threads take several groups of rows each: 8.1 M rows FP64
+// 83.5 us a launch, 86.8 with a block per 2,048 rows.
 static int update_grid(int n, int R) { return std::max(1, std::min(div_up(div_up(n, R), kUpdateThreads), kUpdateGrid)); }
 
 // Launches iteration k of a chunk (SpMV kernel, update kernel); with profiling on,
@@ -1162,7 +1160,7 @@ static int read_state(const CgState* st, HostState* h, hipStream_t s) {
 }
 
 // ------------------------------------------------- CG chunks as HIP graphs
-// On small systems an iteration's three kernels take a few microseconds each,
+// On small systems an iteration's two kernels take a few microseconds each,
 // and launching them from the host costs more than running them.  There a
 // chunk of kGraphIters iterations is captured once into a HIP graph (on a
 // private stream: the caller's may be the null stream, which cannot be
@@ -1387,7 +1385,6 @@ static void minres_layout(Work& w, int n, MinresBufs& B) {
   B.r1 = w.take<double>(n);
   B.r2 = w.take<double>(n);
   B.wv = w.take<double>(n);
-  w.take<double>(n);  // unused; workspaces keep their size
   B.w2 = w.take<double>(n);
 }
 
