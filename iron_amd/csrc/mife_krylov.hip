@@ -41,7 +41,9 @@ constexpr int kFinThreads = 1024;  // one-block finishers (up to kRedBlocks part
 constexpr int kUpdateThreads = 1024;
 constexpr int kMaxIterChunk = 256;  // CG iterations launched between two host reads of the state
 
-struct CgScalars {
+// A cache line of its own per slot: what block 0 of a launch stores lies in no line that
+// the others read.
+struct alignas(128) CgScalars {
   double rz, beta, rr, bb, tol2;
   double rz_prev, rr_seg, rr64;  // rr_seg: recurrence r.r when a segment ended
   // Segmented (mixed-precision) solves: a segment pauses once r.r <= seg_rr, set at

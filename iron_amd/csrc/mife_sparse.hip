@@ -79,9 +79,13 @@ __global__ void sell_build_kernel(int n, const int32_t* __restrict__ rp, const i
 // apart so that a boundary plane's rows spread over many blocks; each wavefront forms
 // src + rhs of one run, one row per lane, and lists the rows that take a lifting
 // term; then 16 lanes walk each listed row, 16 rows side by side, four entries in
-// flight per lane.  75 x 83 x 67 nodes, source and every face fixed: 197 us with
-// the listed rows of 64 walked by one wavefront one by one, 75 us with each fixed
-// entry's loads behind its own test, 38 us now.
+// flight per lane.  75 x 83 x 67 triquadratic nodes, source and every face fixed: 197 us
+// with the listed rows of 64 walked by one wavefront one by one, 75 us with each fixed
+// entry's loads behind its own test, 38 us now.  Without rhs_fixed flags (allowed; the
+// server passes none) every row is listed and 12 B instead of 4 are read of an entry that
+// is not fixed; walked one by one -> now, two faces fixed: 108 -> 110 us there, 97^3 nodes
+// 268 -> 248, 90^3 trilinear nodes 143 -> 76, 97 x 33 x 33 elasticity nodes 110 -> 101,
+// 1001^2 plane nodes 166 -> 87.
 constexpr int kRhsRows = 256;
 
 __global__ __launch_bounds__(256) void solver_rhs_kernel(int n_free, const int32_t* __restrict__ free_idx,
