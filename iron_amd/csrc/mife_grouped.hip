@@ -37,8 +37,9 @@
 // wavefronts of a block sharing a SELL3 slice and the sums formed during the product
 // (all sixteen active: product 127 -> 107 us; the last 139 MB one alone: 29.5 -> 25.9).
 // One wavefront per SELL3 slice with the sums formed during the product: 188.4 ms.
-// A stream of 1,024 requests, 256 at a time: 43.6 -> 48.2 solves/s with mixed requests,
-// 74.8 -> 77.0 with FP64 ones.
+// One 3,600-slice elasticity request alone: sell3_slices.  A stream of 640 requests, 256 at a
+// time, is bound by its large elasticity matrices: 78 solves/s FP64 before and after, 40 to 45
+// in mixed precision.
 #include "mife_common.hpp"
 #include "mife_profile.hpp"
 #include "mife_sparse.hpp"

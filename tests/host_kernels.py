@@ -1,4 +1,4 @@
-"""Compiles device code of iron_amd/csrc for the CPU (tests/host_shim: one block at a
+"""Compiles device code of iron_amd/csrc for the CPU (tests/cpu_block: one block at a
 time, a fiber per thread) and runs a C++ main over it."""
 import re
 import shutil
@@ -9,7 +9,7 @@ import pytest
 
 ROOT = Path(__file__).resolve().parent.parent
 CSRC = ROOT / "iron_amd" / "csrc"
-SHIM = ROOT / "tests" / "host_shim"
+CPU_BLOCK = ROOT / "tests" / "cpu_block"
 CLANG = next((c for c in ("/opt/rocm/llvm/bin/clang++", shutil.which("clang++")) if c and Path(c).exists()), None)
 
 
@@ -34,7 +34,7 @@ def definition(name, what):
 
 
 def _no_launches(text):
-    """Host launch statements become plain calls (main launches through the shim)."""
+    """Host launch statements become plain calls (main launches through the header)."""
     return re.sub(r"<<<.*?>>>", "", text, flags=re.S)
 
 
@@ -46,7 +46,7 @@ def build(tmp_path, source, main, *flags):
     for h in CSRC.glob("*.hpp"):
         (tmp_path / h.name).write_text(_no_launches(h.read_text().replace("../../include", str(ROOT / "include"))))
     src.write_text(_no_launches(source) + main)
-    r = subprocess.run([CLANG, "-std=c++20", "-O1", "-w", *flags, f"-I{SHIM}", str(src), "-o", str(exe)],
+    r = subprocess.run([CLANG, "-std=c++20", "-O1", "-w", *flags, f"-I{CPU_BLOCK}", str(src), "-o", str(exe)],
                        capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-4000:]
     return exe
