@@ -776,15 +776,14 @@ __global__ __launch_bounds__(8 * E * G) void scalar_batch_kernel(const BatchJob*
   }
 }
 
-template <typename T>
+template <typename T, int TURNS>
 __global__ __launch_bounds__(256) void elastic_batch_kernel(const BatchJob* __restrict__ jobs,
                                                             const BatchSeg* __restrict__ segs, int nseg, int total,
-                                                            int turns,
                                                             const double* __restrict__ dN,
                                                             const double* __restrict__ w) {
-  for (int base = blockIdx.x * 4 * turns; base < total; base += gridDim.x * 4 * turns) {
+  for (int base = blockIdx.x * 4 * TURNS; base < total; base += gridDim.x * 4 * TURNS) {
     const int slot = q1_elastic_slot(), idx = base + slot;
-    const bool active = slot < 4 * turns && idx < total;
+    const bool active = slot < 4 * TURNS && idx < total;
     ElasticJob<T> J{};
     long long e = 0;
     if (active) {
@@ -793,7 +792,7 @@ __global__ __launch_bounds__(256) void elastic_batch_kernel(const BatchJob* __re
       J = ElasticJob<T>{B.coords, B.enodes, B.coef, B.pos, (T*)B.vals, 0, 0};
       e = B.order[sg.begin + idx - sg.prefix];
     }
-    q1_elastic_elements<T, false>(J, e, active, turns, dN, w, false);
+    q1_elastic_elements<T, false>(J, e, active, TURNS, dN, w, false);
   }
 }
 
@@ -820,10 +819,16 @@ static void q1_scalar_launch(long long count, F&& f) {
 // (at 8 all its blocks are resident), 61 x 47 x 53 1203 / 1055 / 1030 / 1114.  FP32 holds more
 // wavefronts: 45^3 375 / 389 / 353 / 366, 61 x 47 x 53 609 / 600 / 641 / 574.  Atomic adds
 // bound the atomic form: 1224 / 1236 / 1215 / 1261 there, FP32 951 / 954 / 957 / 962.
-enum class Form { kStage, kColour, kAtomic };
+// Batches (many meshes, a colour of all to a launch; the number is a constant of their
+// kernels, as a variable it cost 10%): 8 meshes of 8^3, 512 to a launch, 87 / 101 / 133 /
+// 200, 16 of 12^3 (3,456) 232 / 188 / 206 / 261, 4 of 24^3 (6,912) 415 / 350 / 324 / 348,
+// 2 of 60^3 (54,000) 3378 / 3334 / 3343 / 3352, FP32 2136 / 1905 / 1792 / 1850.
+enum class Form { kStage, kColour, kAtomic, kBatch };
 template <typename T>
 static int elastic_turns(long long count, Form form) {
   if (form == Form::kAtomic) return sizeof(T) == 4 || count < 8192 ? 1 : 4;
+  if (form == Form::kBatch)
+    return count < 1024 ? 1 : count < 6144 ? 2 : sizeof(T) == 8 || count < 16384 ? 4 : 8;
   if (form == Form::kStage) return count < 1024 ? 1 : count < 4096 ? 2 : count < 8192 ? 4 : 8;
   if (sizeof(T) == 4) return count < 4096 ? 1 : count < 8192 ? 2 : count < 16384 ? 4 : 8;
   return count < 4096 ? 1 : count < 8192 ? 2 : count < 16384 ? 8 : 4;
@@ -1324,23 +1329,34 @@ extern "C" int mife_assemble_batch(const mife_element_desc* scalar_desc, const m
   const BatchSeg* ds = (const BatchSeg*)((char*)work + align256(sizeof(BatchJob) * n_jobs));
   const int tk = prof::begin(s);
   for (const Launch& L : launches) {
-    auto grid = [&](int per) { return std::max(1, std::min(div_up(L.total, per), kBatchGrid)); };
+    // blocks of `per` elements and `waves` wavefronts, as many as are resident
+    auto grid = [&](int per, int waves) {
+      return std::max(1, std::min(div_up(L.total, per), kBatchGrid * 4 / waves));
+    };
     if (L.kind == MIFE_JOB_SCALAR) {
       q1_scalar_launch(L.total, [&](auto per, auto groups) {
         constexpr int E = decltype(per)::value, G = decltype(groups)::value;
         if (prec == MIFE_F64)
-          scalar_batch_kernel<double, E, G><<<grid(E), 8 * E * G, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, scalar_desc->dN,
+          scalar_batch_kernel<double, E, G><<<grid(E, E * G / 8), 8 * E * G, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, scalar_desc->dN,
                                                                    scalar_desc->N, scalar_desc->w);
         else
-          scalar_batch_kernel<float, E, G><<<grid(E), 8 * E * G, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, scalar_desc->dN,
+          scalar_batch_kernel<float, E, G><<<grid(E, E * G / 8), 8 * E * G, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, scalar_desc->dN,
                                                                   scalar_desc->N, scalar_desc->w);
       });
     } else {
       auto elastic = [&](auto zero) {
         using T = decltype(zero);
-        const int turns = elastic_turns<T>(L.total, Form::kColour);
-        elastic_batch_kernel<T><<<grid(4 * turns), 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total, turns,
-                                                                elastic_desc->dN, elastic_desc->w);
+        auto go = [&](auto turns) {
+          constexpr int TURNS = decltype(turns)::value;
+          elastic_batch_kernel<T, TURNS><<<grid(4 * TURNS, 4), 256, 0, s>>>(dj, ds + L.seg0, L.nseg, L.total,
+                                                                            elastic_desc->dN, elastic_desc->w);
+        };
+        switch (elastic_turns<T>(L.total, Form::kBatch)) {
+          case 1: go(std::integral_constant<int, 1>{}); break;
+          case 2: go(std::integral_constant<int, 2>{}); break;
+          case 4: go(std::integral_constant<int, 4>{}); break;
+          default: go(std::integral_constant<int, 8>{}); break;
+        }
       };
       if (prec == MIFE_F64) elastic(0.0);
       else elastic(0.0f);

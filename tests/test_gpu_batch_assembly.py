@@ -85,3 +85,40 @@ def test_batch_equals_per_mesh_assembly():
             assert torch.equal(ref[k], out[k]), (prec, shapes[k])
             if ref_s[k] is not None:
                 assert torch.equal(ref_s[k], out_s[k]), (prec, shapes[k])
+
+
+@pytest.mark.parametrize("kind,shapes", [
+    ("elasticity", [(20, 20, 20)]), ("elasticity", [(12, 11, 10), (18, 20, 19)]), ("elasticity", [(36, 37, 37)]),
+    ("elasticity", [(51, 51, 51)]), ("diffusion", [(25, 25, 26)]), ("diffusion", [(18, 18, 18), (20, 29, 20)]),
+    ("diffusion", [(122, 119, 111), (3, 2, 5)])])
+def test_batch_launch_shapes(kind, shapes):
+    """Launches about the element counts from which more elements go to a wavefront or a
+    block (1,024, 6,144 and 16,384 elasticity elements, 2,048 and 200,000 scalar ones; a
+    launch holds an eighth of the batch): each mesh as by its own assembly, bit for bit."""
+    from iron_amd import _lib, fem
+    from iron_amd.basis import basis
+    sts = [_Mesh(kind, ne) for ne in shapes]
+    q1 = fem.DeviceBasis(basis(3, 1, 2), "cuda")
+    d = C.byref(q1.desc)
+    L = _lib.lib()
+    for prec in (fem.F64, fem.F32):
+        print(f"case batch {kind} {shapes} prec={prec}", flush=True)
+        coefs = [st.coefficients(50 + i, "cuda") for i, st in enumerate(sts)]
+        ref = [st.asm.assemble(st.csr.zeros(prec), cf, prec=prec) for st, cf in zip(sts, coefs)]
+        out = [st.csr.zeros(prec) for st in sts]
+        jobs = (_lib.AssemblyJob * len(sts))()
+        for k, st in enumerate(sts):
+            cs, asm = st.csr, st.asm
+            jobs[k] = _lib.AssemblyJob(_lib.MIFE_JOB_SCALAR if kind == "diffusion" else _lib.MIFE_JOB_ELASTIC,
+                                       asm.n_elem, _lib.ptr(asm.coords), _lib.ptr(asm.elem_nodes),
+                                       _lib.ptr(cs.elem_dofs), _lib.ptr(coefs[k]), None, _lib.ptr(cs.pos),
+                                       _lib.ptr(cs.order), cs.colour_ptr.ctypes.data, cs.n_colours, 0,
+                                       _lib.ptr(out[k]), None)
+        maxc = max(st.csr.n_colours for st in sts)
+        nb = int(L.mife_assemble_batch_work_bytes(len(sts), maxc))
+        host, dev = np.empty(nb, dtype=np.uint8), torch.empty(nb, dtype=torch.uint8, device="cuda")
+        _lib.call("mife_assemble_batch", d, d, len(sts), jobs, maxc, prec, host.ctypes.data, _lib.ptr(dev),
+                  _lib.stream_ptr())
+        torch.cuda.synchronize()
+        for k in range(len(sts)):
+            assert torch.count_nonzero(ref[k]) > 0 and torch.equal(ref[k], out[k]), (prec, shapes[k])
